@@ -1,292 +1,338 @@
 // The qkv linear fused with the self-attention epilogue and the head-major
-// pack (t2h_qkv_linear_pack), on the GEMM core (tiling and pipeline:
-// t2h_gemm_core.h): a wave's 128 features are one head of 128 or two heads of
-// 64. T2H_QKV_WAVES picks
-// the layout: 8 (shipped; 64 tokens per wave, 128 accumulators, 10 % faster
-// on the config-5 qkv) or 4 (128 tokens per wave, direct-to-LDS loads).
+// pack (t2h_qkv_linear_pack), on the persistent main loop of t2h_gemm_core.h:
+// a wave's 128 features are one head of 128 or two heads of 64.
 //
 // Reference: the qkv enqueue_gemm + bias_rms_rope_qkv + pack_q_z + pack_kv_z
 // of the self-attention chain (gpu/attention.mojo:507-563, 566-594, 634-662,
 // sequence 983-1013).
-#ifndef T2H_QKV_WAVES
-#define T2H_QKV_WAVES 8
-#endif
-#define T2H_GEMM_WAVES T2H_QKV_WAVES
 #include "t2h_gemm_core.h"
 
 namespace t2h {
 namespace {
 
 // ---- qkv linear + attention epilogue + head-major pack ----------------------
-// The qkv GEMM's output [rows, 3, H, HD] never reaches memory. A wave's 128
-// features are one head of HD = 128 or two heads of HD = 64 (q, k or v: head
-// hg = n / HD, tensor hg / H, head hg % H) for kWT tokens (64 with 8 waves,
-// 128 with 4), and each token's head lives in two lanes (l and l ^ 32, 64 or
-// 32 values each: the MFMA tile of feature tile fi holds features fi*32 +
-// 8q + 4h + i in lane half h). Per token, in the
-// order of the separate kernels
-// (bias_rms_rope_qkv, pack_q_z, pack_kv_z): + bias; q/k: RMS over the head,
-// x * rsqrt(sum x^2) * (gamma * sqrt(D)); q/k: RoPE on the in-lane pairs
-// (2p, 2p + 1) with cos/sin from the phase table or from the token's
-// position; q: * 1/sqrt(D); tokens >= rows: 0. The head then goes through
-// the wave's own LDS region (kStaged tokens at a time: 64 with 4 waves, 32
-// with 8, 16 KB or 8 KB) as 256-byte token rows (one or two heads) and
-// leaves as 16-byte vectors: whole token rows of each head (qh [H, mp, D],
-// k [H, lp, D], vh [H, lp, D]) or, for the transposed k [H, D, lp], 8 tokens
-// of one feature gathered from 8 rows. Tiles past the last token row skip the
-// GEMM and write the pads.
-constexpr int kHead = 128;   // features of a wave (one staged token row: 256 bytes of 16-bit values)
-static_assert(kTJ == 2 || kTJ == 4, "copy_col cases");
-constexpr int kStaged = kWaves == 8 ? 32 : 64;   // token rows a wave stages at a time
-constexpr int kJJ = kStaged / 32;                // token tiles per staged group
-constexpr int kRegion = kStaged * 256;           // bytes of a wave's staging region
-constexpr int kParamOff = kWaves * kRegion;      // [head][bias, gamma * sqrt(D)][128] f32
-constexpr int kPPT = 2 * 2 * kHead / kGemmThreads;   // parameters per thread
-// 8 waves unroll their two groups, so that each group's accumulators are used
-// in place and are dead after it (128 accumulators in 256 registers); 4 waves
-// keep the loop (a runtime token tile picks its accumulators by a switch).
-constexpr int kGrpUnroll = kWaves == 8 ? kTJ / kJJ : 1;
+// The qkv GEMM's output [rows, 3, H, HD] never reaches memory. A tile's 256
+// features lie in one of q, k and v (H * HD is a multiple of 256). Per token,
+// in the order of the separate kernels (bias_rms_rope_qkv, pack_q_z,
+// pack_kv_z): + bias; q/k: RMS over the head, x * rsqrt(sum x^2) * (gamma *
+// sqrt(D)); q/k: RoPE on the in-lane pairs (2p, 2p + 1) with cos/sin from the
+// phase table or from the token's position; q: * 1/sqrt(D); tokens >= rows: 0.
+// A token's head lies in the four lanes l, l ^ 16, l ^ 32, l ^ 48.
+//
+// cos/sin from positions: computing them per head and token (64 sincosf per
+// token and head) took 395 us of the 3,243 us of 201,436 tokens x 4608
+// features. Voxel coordinates are small integers, so each block computes
+// cos/sin of every (position < kPos, frequency) once, into LDS, with the same
+// sincosf of the same f32 angle, and its tiles look them up; a token outside
+// the table takes the direct computation.
+//
+// The values leave as whole 128-byte row pieces: through 2 KB of LDS per wave
+// (16 tokens x 64 features) for qh [H, mp, D], k [H, lp, D], vh [H, lp, D];
+// for the transposed k [H, D, lp] through the wave's share of the two stages,
+// where 8 tokens of one feature are gathered per lane (such a tile requests
+// the next tile's operands only afterwards). Tiles past the last token row
+// skip the GEMM and write the pads.
+constexpr int kHead = 128;                     // features of a wave
+constexpr int kPos = 128;                      // positions of the cos/sin table, where they fit
+// LDS past the stages: [wave half][bias, gamma * sqrt(D)][128] f32, the tile's
+// packed positions, the slots' table columns, the table
+constexpr int kPosOff = 2048, kSlotOff = kPosOff + 1024, kTabOff = kSlotOff + 256, kExtra = 32768;
+constexpr int kTabEntries = (kExtra - kTabOff) / 8;
+constexpr uint32_t kNoPos = 0xFFFFFFFFu;       // a token whose position is not in the table
 
 // Slot of a 16-byte chunk in a staged 256-byte token row: chunk c of row r
-// at c ^ stage_swz(r). Over 32 consecutive rows (one row-major write) every
-// slot appears twice; over rows 8g + j, g = 0..7 (one transposed gather)
-// the slots are distinct; a row's 16 chunks are a permutation.
+// at c ^ stage_swz(r). Over 16 consecutive rows (one write) every slot appears
+// once; over rows 8g + j, g = 0..7 (one transposed gather) the slots are
+// distinct; a row's 16 chunks are a permutation.
 __device__ __forceinline__ int stage_swz(int r) { return ((r >> 3) ^ ((r & 7) << 1)) & 15; }
 
-template <int TJ>
-__device__ __forceinline__ void copy_col(const f32x16 (&acc)[kFI][kTJ], float (&col)[kFI][16]) {
-#pragma unroll
-    for (int fi = 0; fi < kFI; ++fi)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) col[fi][r] = acc[fi][TJ][r];
-}
-
-template <typename T, bool KT, int HD>
-__global__ __launch_bounds__(kGemmThreads, T2H_GEMM_OCC) void qkv_pack_kernel(GemmArgs g, PackArgs p, RopeSlots tab) {
+template <typename T, bool KT, int HD, int BT, bool W64>
+__global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackArgs p, RopeSlots tab) {
+    constexpr int kTJ = Big<BT>::kTJ;
     constexpr int NH = kHead / HD;    // heads per wave
-    constexpr int FPH = kFI / NH;     // 32-feature MFMA tiles per head
-    constexpr int CPH = HD / 8;       // 16-byte chunks of a head's token row
-    // One LDS array: the GEMM's stages, then the epilogue's staging (a
-    // region per wave) and the tile's parameters at 64 KB. (A separate
-    // parameter array that took the kernel past 128 KB of LDS measured 20 %
-    // slower on MI355X.)
-    __shared__ __attribute__((aligned(1024))) uint8_t lds[kStages * kStageBytes];
-    static_assert(kWF == kHead && kHead % HD == 0 && kFI % NH == 0 && kWT % kStaged == 0 &&
-                      kParamOff + 2 * 2 * kHead * 4 <= kStages * kStageBytes,
-                  "staging layout");
-    static_assert(kPPT * kGemmThreads == 2 * 2 * kHead, "parameters per thread");
-    TileOf tile;
-    if (!tile.init(g)) return;
-    const int64_t t0 = tile.t0, n0 = tile.n0;
+    constexpr int FPH = 8 / NH;       // 16-feature MFMA tiles per head
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[2 * Big<BT>::kStage + kExtra];
+    TileWalk walk(g);
+    if (!walk.more()) return;
+    BigCtx<BT, W64> c;
+    c.init(g, lds);
+    const int steps = g.k / kBK;
+    const int wave = c.wave;
+    const int wf = wave >> 2, wt = wave & 3;
+    uint8_t* extra = lds + 2 * Big<BT>::kStage;
+    const float* pb = reinterpret_cast<const float*>(extra) + (wf * 2 + 0) * kHead;
+    const float* pg = reinterpret_cast<const float*>(extra) + (wf * 2 + 1) * kHead;
+    const bool lookup = p.use_rope && p.phases == nullptr && g.rows > 0;
+    const int fd = p.freq_dim;
+    const int npos = fd > 0 ? (kTabEntries - 1) / fd < kPos ? (kTabEntries - 1) / fd : kPos : 0;
 
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    const int wf = wave & 1, wt = wave >> 1;
-    const int fr = lane & 31, h = lane >> 5;
-    const int hg = (int)((n0 + wf * kWF) / HD);
-    const int which = hg / p.heads;          // 0 q, 1 k, 2 v (the wave's heads share it: 128 | H * HD)
-    const int z = hg - which * p.heads;      // the wave's first head
-    const float* __restrict__ bias = which == 0 ? p.bias_q : which == 1 ? p.bias_k : p.bias_v;
-    const float* __restrict__ gamma = which == 0 ? p.gamma_q : which == 1 ? p.gamma_k : nullptr;
-
-    // the tile's bias and gamma * sqrt(D) (slot i = (wave group * 2 + kind) *
-    // 128 + d, kPPT slots per thread; a group's 128 features are consecutive
-    // in the [H * HD] parameter rows) are requested before the GEMM and land
-    // in LDS after it
-    float pv[kPPT];
-#pragma unroll
-    for (int j = 0; j < kPPT; ++j) {
-        const int i = (int)threadIdx.x + j * kGemmThreads;
-        const int ph = i / (2 * kHead), kind = (i / kHead) & 1, pd = i % kHead;
-        const int hp = (int)((n0 + ph * kWF) / HD);
-        const int wp = hp / p.heads;
-        const int pz = hp - wp * p.heads;
-        const float* src = kind == 0 ? (wp == 0 ? p.bias_q : wp == 1 ? p.bias_k : p.bias_v)
-                                     : (wp == 0 ? p.gamma_q : wp == 1 ? p.gamma_k : nullptr);
-        pv[j] = src != nullptr ? src[pz * HD + pd] : 0.0f;
+    int64_t tt, ft;
+    tile_at(g, walk.lo + walk.i, tt, ft);
+    if (tt * BT < g.rows) {
+        c.tile(g, tt * BT, ft * kBF);
+        c.prologue(steps);
     }
-    f32x16 acc[kFI][kTJ];
-    zero_acc(acc);
-    if (t0 < g.rows) gemm_mainloop<T>(g, t0, n0, lds, acc);   // block-uniform (ends with a barrier)
-    float* prm = reinterpret_cast<float*>(lds + kParamOff);
-#pragma unroll
-    for (int j = 0; j < kPPT; ++j) {
-        const int i = (int)threadIdx.x + j * kGemmThreads;
-        prm[i] = ((i / kHead) & 1) ? pv[j] * p.rms_scale : pv[j];
+    if (lookup) {
+        // entry pos * fd + f: (cos, sin); the last entry is the identity. A
+        // slot's word: its column's byte offset | axis << 16 (4: none)
+        float2* t = reinterpret_cast<float2*>(extra + kTabOff);
+        for (int e = threadIdx.x; e < npos * fd; e += kThreads) {
+            const float pos = (float)(e / fd);
+            float cv, sv;
+            slot_phase(&pos, 0, tab.freq[e % fd], cv, sv);
+            t[e] = float2{cv, sv};
+        }
+        if (threadIdx.x == 0) t[npos * fd] = float2{1.0f, 0.0f};
+        if (threadIdx.x < HD / 2) {
+            const int ax = slot_axis(threadIdx.x, fd, p.pos_dim);
+            reinterpret_cast<uint32_t*>(extra + kSlotOff)[threadIdx.x] =
+                ax < 0 ? (uint32_t)(npos * fd * 8) | (4u << 16) : (uint32_t)((threadIdx.x - ax * fd) * 8) | (ax << 16);
+        }
+        wait_lds();
     }
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    __builtin_amdgcn_s_barrier();
-
-    const bool rope = p.use_rope && which < 2 && g.rows > 0;
-    const int64_t extent = which == 0 ? p.mp : p.lp;
-    T* __restrict__ out = static_cast<T*>(which == 0 ? p.qh : which == 1 ? p.k_out : p.vh);
-    const bool trans = KT && which == 1;
-    uint8_t* region = lds + wave * kRegion;
-    const float* pb = prm + (wf * 2 + 0) * kHead;
-    const float* pg = prm + (wf * 2 + 1) * kHead;
-
-#pragma unroll kGrpUnroll
-    for (int grp = 0; grp < kTJ / kJJ; ++grp) {
-#pragma unroll kGrpUnroll
-        for (int jj = 0; jj < kJJ; ++jj) {
-            const int tj = grp * kJJ + jj;
-            // this token tile's accumulators (static register indices per case)
-            float col[kFI][16];
-            switch (tj) {
-                case 0: copy_col<0>(acc, col); break;
-                case 1: copy_col<1>(acc, col); break;
-                case 2: copy_col<(kTJ > 2 ? 2 : 0)>(acc, col); break;
-                default: copy_col<(kTJ > 2 ? 3 : 1)>(acc, col); break;
+    while (true) {
+        const int64_t t0 = tt * BT, n0 = ft * kBF;
+        const int hg = (int)(n0 / HD);
+        const int which = hg / p.heads;          // 0 q, 1 k, 2 v
+        const int z = hg - which * p.heads + wf * NH;      // the wave's first head
+        const float* __restrict__ bias = which == 0 ? p.bias_q : which == 1 ? p.bias_k : p.bias_v;
+        const float* __restrict__ gamma = which == 0 ? p.gamma_q : which == 1 ? p.gamma_k : nullptr;
+        const bool rope = p.use_rope && which < 2 && g.rows > 0;
+        // one bias or gamma value and one token's position per thread, read
+        // ahead of the main loop and staged in LDS after it
+        float pv;
+        {
+            const int i = threadIdx.x, f = (hg - which * p.heads) * HD + (i >> 8) * kHead + (i & 127);
+            const float* src = (i >> 7) & 1 ? gamma : bias;
+            pv = src != nullptr ? src[f] : 0.0f;
+            if ((i >> 7) & 1) pv *= p.rms_scale;
+        }
+        uint32_t pw = kNoPos;
+        if (rope && lookup && threadIdx.x < BT) {
+            const int64_t t = t0 + threadIdx.x < g.rows ? t0 + threadIdx.x : g.rows - 1;
+            const PosSource src{p.coords, p.coord_cols, p.grid_res, p.pos_dim};
+            float pos[T2H_MAX_POS_DIM];
+            src.get(t, pos);
+            bool in = true;
+            uint32_t w = 0;
+#pragma unroll
+            for (int ax = 0; ax < T2H_MAX_POS_DIM; ++ax) {
+                in = in && pos[ax] >= 0.0f && pos[ax] < (float)npos;
+                w |= ((uint32_t)(int)pos[ax] & 0xFFu) << (8 * ax);
             }
-            const int tl = jj * 32 + fr;                      // staged row (token within the group)
-            const int64_t t = t0 + wt * kWT + tj * 32 + fr;
+            pw = in ? w : kNoPos;
+        }
+        f32x4 acc[8][kTJ];
+        if (t0 < g.rows) {
+            big_mainloop<T, BT, W64>(c, steps, acc);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+#pragma unroll
+                for (int j = 0; j < kTJ; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            turn_barrier();      // the last tile's LDS is read
+        }
+        const int lane = fresh_lane(c.lane);
+        const int fr = lane & 15, h = lane >> 4;
+        walk.i += walk.per;
+        const bool more = walk.more();
+        if (more) tile_at(g, walk.lo + walk.i, tt, ft);
+        const bool next = more && tt * BT < g.rows;
+        const bool trans = KT && which == 1;
+        if (next) {
+            c.tile(g, tt * BT, ft * kBF);
+            if (!trans) c.prologue(steps);
+        }
+        reinterpret_cast<float*>(extra)[threadIdx.x] = pv;
+        if (threadIdx.x < BT) reinterpret_cast<uint32_t*>(extra + kPosOff)[threadIdx.x] = pw;
+        wait_lds();
+        turn_barrier();
+
+        const int64_t extent = which == 0 ? p.mp : p.lp;
+        T* __restrict__ out = static_cast<T*>(which == 0 ? p.qh : which == 1 ? p.k_out : p.vh);
+        const int64_t tw = t0 + wt * Big<BT>::kWT;
+        uint8_t* region = trans ? lds + wave * (Big<BT>::kWT * 256) : lds + Big<BT>::kSpare + wave * 2048;
+        // + bias and the RMS, in place: feature tiles outside, so that each
+        // parameter is read once
+        float ss[NH][kTJ];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const f32x4 b4 = *reinterpret_cast<const f32x4*>(pb + i * 16 + h * 4);
+#pragma unroll
+            for (int j = 0; j < kTJ; ++j) {
+                float v[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[e] = bias != nullptr ? add_rn(acc[i][j][e], b4[e]) : acc[i][j][e];
+                const float q = sum_sq<4>(v);
+                ss[i / FPH][j] = i % FPH == 0 ? q : ss[i / FPH][j] + q;
+                acc[i][j] = f32x4{v[0], v[1], v[2], v[3]};
+            }
+        }
+        if (gamma != nullptr) {
+#pragma unroll
+            for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+                for (int j = 0; j < kTJ; ++j) {
+                    float q = ss[hh][j];
+                    q += __shfl_xor(q, 16);
+                    q += __shfl_xor(q, 32);
+                    ss[hh][j] = q < 1e-24f ? 1e12f : __builtin_amdgcn_rsqf(q);
+                }
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const f32x4 g4 = *reinterpret_cast<const f32x4*>(pg + i * 16 + h * 4);
+#pragma unroll
+                for (int j = 0; j < kTJ; ++j)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[i][j][e] = (acc[i][j][e] * ss[i / FPH][j]) * g4[e];
+            }
+        }
+        // 16 tokens x 64 features at a time: RoPE, q's scale, pads, out
+#pragma unroll
+        for (int j = 0; j < kTJ; ++j) {
+            const int64_t t = tw + j * 16 + fr;
             const int64_t tc = t < g.rows ? t : g.rows - 1;   // clamped for position reads
             const bool live = t < g.rows;
-            // feature of col[fi][4q + i]: d = fi*32 + 8q + 4h + i
-            // the token's cos/sin (table path) are requested first and arrive
-            // while the bias and the sum of squares are computed
-            float cs[kFI][4][4];
-            const bool table = rope && p.phases != nullptr;
-            if (table) {
-                const float* row = p.phases + (tc % p.phase_rows) * HD;
+            uint32_t pos = kNoPos;
+            if (rope && lookup) pos = reinterpret_cast<const uint32_t*>(extra + kPosOff)[wt * Big<BT>::kWT + j * 16 + fr];
+            const bool direct = rope && lookup && __any(pos == kNoPos);
 #pragma unroll
-                for (int fi = 0; fi < kFI; ++fi)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) load_params<4>(row + (fi % FPH) * 32 + q * 8 + h * 4, cs[fi][q]);
-            }
-            if (bias != nullptr) {
-#pragma unroll
-                for (int fi = 0; fi < kFI; ++fi)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float4 b4 = *reinterpret_cast<const float4*>(pb + fi * 32 + q * 8 + h * 4);
-                        col[fi][q * 4 + 0] = add_rn(col[fi][q * 4 + 0], b4.x);
-                        col[fi][q * 4 + 1] = add_rn(col[fi][q * 4 + 1], b4.y);
-                        col[fi][q * 4 + 2] = add_rn(col[fi][q * 4 + 2], b4.z);
-                        col[fi][q * 4 + 3] = add_rn(col[fi][q * 4 + 3], b4.w);
-                    }
-            }
-            // each head's sum of squares: HD / 2 values here, HD / 2 in lane ^ 32
-            float rn[NH];
-#pragma unroll
-            for (int hh = 0; hh < NH; ++hh) rn[hh] = 1.0f;
-            if (gamma != nullptr) {
-#pragma unroll
-                for (int hh = 0; hh < NH; ++hh) {
-                    float ss = 0.0f;
-#pragma unroll
-                    for (int fi = hh * FPH; fi < (hh + 1) * FPH; ++fi) ss += sum_sq<16>(col[fi]);
-                    ss += __shfl_xor(ss, 32);
-                    rn[hh] = ss < 1e-24f ? 1e12f : __builtin_amdgcn_rsqf(ss);
-                }
-            }
-            float pos[T2H_MAX_POS_DIM];
-            if (rope && !table) {
-                const PosSource src{p.coords, p.coord_cols, p.grid_res, p.pos_dim};
-                src.get(tc, pos);
-            }
-#pragma unroll
-            for (int fi = 0; fi < kFI; ++fi) {
-                float* v = col[fi];
-                if (gamma != nullptr) {
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const float4 g4 = *reinterpret_cast<const float4*>(pg + fi * 32 + q * 8 + h * 4);
-                        const float r = rn[fi / FPH];
-                        v[q * 4 + 0] = (v[q * 4 + 0] * r) * g4.x;
-                        v[q * 4 + 1] = (v[q * 4 + 1] * r) * g4.y;
-                        v[q * 4 + 2] = (v[q * 4 + 2] * r) * g4.z;
-                        v[q * 4 + 3] = (v[q * 4 + 3] * r) * g4.w;
-                    }
-                }
+            for (int hf = 0; hf < 2; ++hf) {
+                // cos/sin of the lane's slot pairs: cs[i] = (c, s) of slots s0 + i * 8, + 1
+                const int s0 = (FPH == 8 ? hf * 32 : 0) + h * 2;
+                f32x4 cs[4];
                 if (rope) {
-                    if (table) {
+                    if (!lookup) {
+                        const float* row = p.phases + (tc % p.phase_rows) * HD + s0 * 2;
 #pragma unroll
-                        for (int q = 0; q < 4; ++q) {
-                            rotate_pair(v[q * 4 + 0], v[q * 4 + 1], cs[fi][q][0], cs[fi][q][1]);
-                            rotate_pair(v[q * 4 + 2], v[q * 4 + 3], cs[fi][q][2], cs[fi][q][3]);
+                        for (int i = 0; i < 4; ++i) cs[i] = *reinterpret_cast<const f32x4*>(row + i * 16);
+                    } else if (!direct) {
+                        const uint32_t rowb = (uint32_t)fd * 8;
+                        const uint32_t r0 = (pos & 255) * rowb, r1 = ((pos >> 8) & 255) * rowb,
+                                       r2 = ((pos >> 16) & 255) * rowb, r3 = (pos >> 24) * rowb;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            const u32x2 sw = *reinterpret_cast<const u32x2*>(extra + kSlotOff + (s0 + i * 8) * 4);
+#pragma unroll
+                            for (int q = 0; q < 2; ++q) {
+                                const uint32_t ax = sw[q] >> 16;
+                                const uint32_t ro = ax == 0 ? r0 : ax == 1 ? r1 : ax == 2 ? r2 : ax == 3 ? r3 : 0u;
+                                const float2 v =
+                                    *reinterpret_cast<const float2*>(extra + kTabOff + ro + (sw[q] & 0xFFFFu));
+                                cs[i][2 * q] = v.x;
+                                cs[i][2 * q + 1] = v.y;
+                            }
                         }
                     } else {
+                        const PosSource src{p.coords, p.coord_cols, p.grid_res, p.pos_dim};
+                        float ps[T2H_MAX_POS_DIM];
+                        src.get(tc, ps);
+                        // rolled: unrolled, its sincosf calls crowd the registers of the path that is taken
+#pragma unroll 1
+                        for (int sl = 0; sl < 8; ++sl) {
+                            const int slot = s0 + (sl >> 1) * 8 + (sl & 1);
+                            float cv, sv;
+                            slot_phase(ps, tab.axis[slot], tab.freq[slot], cv, sv);
 #pragma unroll
-                        for (int q = 0; q < 4; ++q)
-#pragma unroll
-                            for (int j = 0; j < 2; ++j) {
-                                const int sl = ((fi % FPH) * 32 + q * 8 + h * 4) / 2 + j;
-                                float c, sn;
-                                slot_phase(pos, tab.axis[sl], tab.freq[sl], c, sn);
-                                rotate_pair(v[q * 4 + 2 * j], v[q * 4 + 2 * j + 1], c, sn);
-                            }
+                            for (int m = 0; m < 8; ++m)
+                                if (m == sl) {
+                                    cs[m >> 1][2 * (m & 1)] = cv;
+                                    cs[m >> 1][2 * (m & 1) + 1] = sv;
+                                }
+                        }
                     }
                 }
 #pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const float x = which == 0 ? mul_rn(v[r], p.q_scale) : v[r];
-                    v[r] = live ? x : 0.0f;
-                }
+                for (int i = 0; i < 4; ++i) {
+                    float v[4];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int c = fi * 4 + q;                  // 16-byte chunk of the 256-byte token row
+                    for (int e = 0; e < 4; ++e) v[e] = acc[hf * 4 + i][j][e];
+                    if (rope) {
+                        rotate_pair(v[0], v[1], cs[i][0], cs[i][1]);
+                        rotate_pair(v[2], v[3], cs[i][2], cs[i][3]);
+                    }
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float x = which == 0 ? mul_rn(v[e], p.q_scale) : v[e];
+                        v[e] = live ? x : 0.0f;
+                    }
                     u32x2 w;
-                    w.x = Word<T>::pack(&v[q * 4]);
-                    w.y = Word<T>::pack(&v[q * 4 + 2]);
-                    *reinterpret_cast<u32x2*>(region + tl * 256 + ((c ^ stage_swz(tl)) * 16) + h * 8) = w;
+                    w.x = Word<T>::pack(v);
+                    w.y = Word<T>::pack(v + 2);
+                    const int ch = i * 2 + (h >> 1);        // 16-byte chunk of the 64 features
+                    const int row = j * 16 + fr;
+                    uint8_t* dst = trans ? region + row * 256 + (((hf * 8 + ch) ^ stage_swz(row)) * 16)
+                                         : region + fr * 128 + ((ch ^ swz(fr)) * 16);
+                    *reinterpret_cast<u32x2*>(dst + (h & 1) * 8) = w;
+                }
+                if (!trans) {        // 64 features: a head of 64, or half of one of 128
+                    wait_lds();
+                    const int64_t zz = HD == 64 ? z + hf : z;
+#pragma unroll
+                    for (int it = 0; it < 2; ++it) {
+                        const int r = it * 8 + (lane >> 3), ch = lane & 7;
+                        const u32x4 w = *reinterpret_cast<const u32x4*>(region + r * 128 + ((ch ^ swz(r)) * 16));
+                        const int64_t to = tw + j * 16 + r;
+                        if (to < extent)
+                            out_store16(out + (zz * extent + to) * HD + (HD == 64 ? 0 : hf * 64) + ch * 8, w);
+                    }
+                    wait_lds();
                 }
             }
         }
-        __builtin_amdgcn_s_waitcnt(0xC07F);      // the wave's LDS writes are done (its region is private)
-        const int64_t tw = t0 + wt * kWT + grp * kStaged;   // first token of the staged rows
-        if (!trans) {
-            // token rows: 16 lanes per 256-byte row, 4 rows per instruction
-#pragma unroll 4
-            for (int it = 0; it < kStaged / 4; ++it) {
-                const int row = it * 4 + (lane >> 4);
-                const int c = lane & 15;
-                const u32x4 w = *reinterpret_cast<const u32x4*>(region + row * 256 + ((c ^ stage_swz(row)) * 16));
-                const int64_t t = tw + row;
-                if (t < extent) out_store16(out + ((int64_t)(z + c / CPH) * extent + t) * HD + (c % CPH) * 8, w);
-            }
-        } else {
-            // feature rows of the transposed k: lane (d, g) gathers feature d
-            // of tokens 8g .. 8g + 7 (eight 2-byte reads, one per token row);
-            // kG groups of 8 tokens, 64 / kG features per instruction
-            constexpr int kG = kStaged / 8;
+        if (trans) {
+            // feature rows of the transposed k: lane (d, gg) gathers feature d of
+            // tokens 8 gg .. 8 gg + 7 (eight 2-byte reads, one per token row)
+            constexpr int kG = Big<BT>::kWT / 8;
+            wait_lds();
 #pragma unroll 2
             for (int it = 0; it < kHead * kG / 64; ++it) {
                 const int d = it * (64 / kG) + lane / kG;
                 const int gg = lane % kG;
                 const int off = (d & 7) * 2;
-                uint32_t wv[4];
+                u32x4 w;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int r0 = gg * 8 + 2 * j, r1 = r0 + 1;
+                for (int q = 0; q < 4; ++q) {
+                    const int r0 = gg * 8 + 2 * q, r1 = r0 + 1;
                     const uint32_t lo = *reinterpret_cast<const uint16_t*>(
                         region + r0 * 256 + (((d >> 3) ^ stage_swz(r0)) * 16) + off);
                     const uint32_t hi = *reinterpret_cast<const uint16_t*>(
                         region + r1 * 256 + (((d >> 3) ^ stage_swz(r1)) * 16) + off);
-                    wv[j] = lo | (hi << 16);
+                    w[q] = lo | (hi << 16);
                 }
-                const int64_t t = tw + gg * 8;
-                if (t < extent) {
-                    u32x4 w;
-                    w.x = wv[0];
-                    w.y = wv[1];
-                    w.z = wv[2];
-                    w.w = wv[3];
-                    out_store16(out + ((int64_t)z * HD + d) * p.lp + t, w);
+                const int64_t to = tw + gg * 8;
+                if (to < extent) {
+                    u32x4* dst = reinterpret_cast<u32x4*>(out + ((int64_t)z * HD + d) * p.lp + to);
+                    if constexpr (BT == 256) __builtin_nontemporal_store(w, dst);    // whole lines
+                    else *dst = w;
                 }
             }
+            wait_lds();
+            turn_barrier();       // every wave has read its share of the stages
+            if (next) c.prologue(steps);
         }
-        // the next group overwrites the staged rows: every lane's reads are done
-        __builtin_amdgcn_s_waitcnt(0xC07F);
+        if (!more) break;
     }
 }
 
-template <typename T, int HD>
-hipError_t qkv_typed(const GemmArgs& g, const PackArgs& p, const RopeSlots& tab, hipStream_t s) {
-    const dim3 grid = grid_1d(g.nblocks), blk(kGemmThreads);
-    if (p.k_transposed) hipLaunchKernelGGL((qkv_pack_kernel<T, true, HD>), grid, blk, 0, s, g, p, tab);
-    else hipLaunchKernelGGL((qkv_pack_kernel<T, false, HD>), grid, blk, 0, s, g, p, tab);
+template <typename T, int HD, int BT, bool W64>
+hipError_t qkv_typed(GemmArgs g, const PackArgs& p, const RopeSlots& tab, int64_t span, hipStream_t s) {
+    g.nblocks = ((span + BT - 1) / BT) * g.ftiles;
+    const dim3 grid = persistent_grid(g.nblocks), blk(kThreads);
+    if (p.k_transposed) hipLaunchKernelGGL((qkv_pack_kernel<T, true, HD, BT, W64>), grid, blk, 0, s, g, p, tab);
+    else hipLaunchKernelGGL((qkv_pack_kernel<T, false, HD, BT, W64>), grid, blk, 0, s, g, p, tab);
     return hipGetLastError();
+}
+
+// 128-token tiles when 256-token ones would occupy half of the CUs at most
+// (each then takes 0.7 of the time: 1,200 tokens x 4608 features on 180 tiles
+// and not 90); 256 otherwise (2,369 tokens: 180 tiles of 256, 33 us; 342 of
+// 128, 45 us).
+template <typename T, int HD>
+hipError_t qkv_sized(const GemmArgs& g, const PackArgs& p, const RopeSlots& tab, int64_t span, hipStream_t s) {
+    if (g.ldx > kMaxStride32 || g.k > kMaxStride32) return qkv_typed<T, HD, 128, true>(g, p, tab, span, s);
+    if ((span + 255) / 256 * g.ftiles * 2 <= device_cu_count()) return qkv_typed<T, HD, 128, false>(g, p, tab, span, s);
+    return qkv_typed<T, HD, 256, false>(g, p, tab, span, s);
 }
 
 }  // namespace
@@ -299,15 +345,14 @@ hipError_t launch_qkv_pack(GemmArgs g, const PackArgs& p, const RopeSlots& tab, 
     if (p.mp > span) span = p.mp;
     if (p.lp > span) span = p.lp;
     g.ftiles = g.n / kBF;
-    g.nblocks = ((span + kBT - 1) / kBT) * g.ftiles;
     g.tgroup = tile_group(g.k);
-    if (g.nblocks == 0) return hipSuccess;
+    if (span == 0) return hipSuccess;
     if (p.head_dim == 64) {
-        if (g.dtype == T2H_F16) return qkv_typed<_Float16, 64>(g, p, tab, s);
-        return qkv_typed<__bf16, 64>(g, p, tab, s);
+        if (g.dtype == T2H_F16) return qkv_sized<_Float16, 64>(g, p, tab, span, s);
+        return qkv_sized<__bf16, 64>(g, p, tab, span, s);
     }
-    if (g.dtype == T2H_F16) return qkv_typed<_Float16, 128>(g, p, tab, s);
-    return qkv_typed<__bf16, 128>(g, p, tab, s);
+    if (g.dtype == T2H_F16) return qkv_sized<_Float16, 128>(g, p, tab, span, s);
+    return qkv_sized<__bf16, 128>(g, p, tab, span, s);
 }
 
 }  // namespace t2h

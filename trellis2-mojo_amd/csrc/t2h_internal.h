@@ -96,6 +96,7 @@ struct PackArgs {
     float q_scale;           // 1 / f32 sqrt(head_dim), baked into qh
     int32_t use_rope;
     int32_t pos_dim;
+    int32_t freq_dim;        // distinct rotary frequencies
     const float* phases;
     int64_t phase_rows;
     const int32_t* coords;
@@ -126,7 +127,7 @@ struct GemmArgs {
     int64_t ldo;
     int32_t out_dtype;       // T2H_F32 or dtype
     int64_t nblocks;         // set by the launcher: token tiles x feature tiles
-    int32_t ftiles;          // feature tiles
+    int32_t ftiles;          // set by the launcher: feature tiles
     int32_t tgroup;          // set by the launcher: token tiles per group of the tile order
     // residual epilogue (t2h_linear_gate_residual): out = res + fl(fl(acc + bias) * gate[b])
     const void* res;         // [rows, n], rows ldo elements apart, out_dtype; may alias out
