@@ -27,12 +27,11 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b16) {
     return __builtin_bit_cast(float, b16 << 16);
 }
 
-// f32 -> bf16 bits, round to nearest even (NaN kept quiet).
+// f32 -> bf16 bits, round to nearest even, NaN kept quiet: v_cvt_pk_bf16_f32,
+// one instruction per pair where the same in integer arithmetic took seven
+// per value (checked equal over all 2^32 inputs).
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
-    uint32_t u = __builtin_bit_cast(uint32_t, f);
-    if ((u & 0x7F800000u) == 0x7F800000u && (u & 0x7FFFFFu)) return (u >> 16) | 0x40u;
-    u += 0x7FFFu + ((u >> 16) & 1u);
-    return u >> 16;
+    return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)f);
 }
 
 __device__ __forceinline__ float f16_bits_to_f32(uint32_t b) {
@@ -67,7 +66,9 @@ template <> struct Word<__bf16> {
         f[1] = __builtin_bit_cast(float, w & 0xFFFF0000u);
     }
     __device__ static __forceinline__ uint32_t pack(const float* f) {
-        return f32_to_bf16_bits(f[0]) | (f32_to_bf16_bits(f[1]) << 16);
+        typedef __bf16 v2 __attribute__((ext_vector_type(2)));
+        const v2 p = {(__bf16)f[0], (__bf16)f[1]};
+        return __builtin_bit_cast(uint32_t, p);
     }
 };
 
