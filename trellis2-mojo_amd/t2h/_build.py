@@ -1,7 +1,8 @@
 """Build recipe for libt2h.so (hipcc, gfx950 only).
 
 Each csrc/*.hip translation unit is compiled in parallel, then linked into
-lib/libt2h.so next to this package. The packed-FP32 target feature is turned
+lib/libt2h.so next to this package; csrc/t2h_pycall.cpp (host code only)
+becomes lib/_t2h_pycall.so, the Python call module. The packed-FP32 target feature is turned
 off for every HIP compile (the host pass warns that it does not know the
 feature; that warning is filtered).
 """
@@ -11,6 +12,7 @@ import concurrent.futures as cf
 import glob
 import os
 import subprocess
+import sysconfig
 
 PKG_ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))   # trellis2-mojo_amd/
 REPO_ROOT = os.path.dirname(PKG_ROOT)
@@ -19,7 +21,9 @@ INCLUDE = os.path.join(REPO_ROOT, "include")
 BUILD_DIR = os.path.join(PKG_ROOT, "_build")
 LIB_DIR = os.path.join(PKG_ROOT, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libt2h.so")
+PYCALL_PATH = os.path.join(LIB_DIR, "_t2h_pycall.so")
 
+CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 CFLAGS = [
@@ -54,6 +58,10 @@ def build(verbose: bool = False) -> str:
     # emitted) fails the link here instead of the first dlopen on a GPU box
     logs.append(_run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,-z,defs", *objs, "-o", tmp]))
     os.replace(tmp, LIB_PATH)
+    tmp = PYCALL_PATH + ".tmp"
+    logs.append(_run([CXX, "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", f"-I{INCLUDE}",
+                      f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "t2h_pycall.cpp"), "-ldl", "-o", tmp]))
+    os.replace(tmp, PYCALL_PATH)
     if verbose:
         print("\n".join(l for l in logs if l.strip()))
     return LIB_PATH

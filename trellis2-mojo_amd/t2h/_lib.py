@@ -2,14 +2,18 @@
 
 The library is loaded once, after torch (so torch's HIP runtime — SONAME
 libamdhip64.so.7 — is the one the library binds to and device pointers are
-shared). There is no fallback: if the library is missing every op raises.
+shared). There is no fallback: if the library or the call module
+(_t2h_pycall.so, the same functions without ctypes' conversions) is missing
+every op raises.
 """
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
-from ._build import LIB_PATH
+from ._build import LIB_PATH, PYCALL_PATH
 
 c_i32, c_i64, c_f32, c_f64, c_p = ctypes.c_int32, ctypes.c_int64, ctypes.c_float, ctypes.c_double, ctypes.c_void_p
 
@@ -68,6 +72,7 @@ _SIGNATURES = {
 EXPORTED = ["t2h_version", "t2h_last_error", "t2h_flow_euler_workspace", *_SIGNATURES]
 
 _lib = None
+_calls = {}     # name -> callable returning the status, filled by load()
 
 
 class T2HError(RuntimeError):
@@ -96,6 +101,13 @@ def load(path: str | None = None):
         fn = getattr(L, name)
         fn.restype = c_i32
         fn.argtypes = args
+    if not os.path.exists(PYCALL_PATH):
+        raise RuntimeError(f"_t2h_pycall.so not found at {PYCALL_PATH}: run __graft_entry__.build() first")
+    loader = importlib.machinery.ExtensionFileLoader("_t2h_pycall", PYCALL_PATH)
+    m = importlib.util.module_from_spec(importlib.util.spec_from_loader("_t2h_pycall", loader))
+    loader.exec_module(m)
+    m.bind(path)
+    _calls.update((name, getattr(m, name, None) or getattr(L, name)) for name in _SIGNATURES)
     _lib = L
     return L
 
@@ -109,4 +121,10 @@ def check(rc: int) -> None:
 
 
 def call(name: str, *args) -> None:
-    check(getattr(load(), name)(*args))
+    f = _calls.get(name)
+    if f is None:
+        load()
+        f = _calls[name]
+    rc = f(*args)
+    if rc != T2H_OK:
+        check(rc)

@@ -140,7 +140,7 @@ class ModulatedCrossBlock:
         m = mod.to(torch.float32).contiguous()
         if m.dim() != 2 or m.shape[1] != 6 * c:
             raise ValueError("ModulatedCrossBlock: mod must be [B, 6C]")
-        return [m[:, i * c:(i + 1) * c] for i in range(6)]
+        return [m.narrow(1, i * c, c) for i in range(6)]
 
     def forward(self, x, mod: torch.Tensor, self_attn: Chain, cross_attn: Chain, mlp: Chain):
         """x: dense [N, L, C] or SparseTensor with feats [T, C]. Returns a new

@@ -24,7 +24,13 @@ OP_ADD, OP_SUB, OP_MUL, OP_DIV, OP_RSUB, OP_RDIV = 0, 1, 2, 3, 4, 5
 
 
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    """torch's current stream on the current device (the handle alone: the
+    Stream object of torch.cuda.current_stream() takes 1.5 us to make)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
+def _ptr(t: Optional[torch.Tensor]):
+    return None if t is None else t.data_ptr()
 
 
 def _dev(t: torch.Tensor, what: str) -> None:
@@ -175,7 +181,7 @@ def _heads_view(t: torch.Tensor, what: str):
     if t.stride(-1) != 1 or t.stride(-2) != d:
         raise ValueError(f"{what}: heads must be contiguous [H, D]")
     lead = t.shape[:-2]
-    rows = int(np.prod(lead)) if len(lead) else 1
+    rows = math.prod(lead)
     if t.dim() == 3:
         stride = t.stride(0)
     else:  # leading dims must collapse to one row stride
@@ -187,7 +193,7 @@ def _heads_view(t: torch.Tensor, what: str):
 
 def _host_freqs(freqs) -> tuple:
     f = np.ascontiguousarray(np.asarray(freqs, dtype=np.float32))
-    return f, (f.ctypes.data if f.size else None), int(f.size)
+    return f, (f.__array_interface__["data"][0] if f.size else None), int(f.size)
 
 
 def qk_rmsnorm_rope(q=None, k=None, gamma_q=None, gamma_k=None, bias_q=None, bias_k=None, freqs=None,
@@ -201,7 +207,7 @@ def qk_rmsnorm_rope(q=None, k=None, gamma_q=None, gamma_k=None, bias_q=None, bia
     rows, h, d, in_stride = _heads_view(ref, "qk_rmsnorm_rope")
     dt = _dtype(ref, "qk_rmsnorm_rope")
     for t in (q, k):
-        if t is not None:
+        if t is not None and t is not ref:
             r2, h2, d2, s2 = _heads_view(t, "qk_rmsnorm_rope")
             if (r2, h2, d2, s2) != (rows, h, d, in_stride) or t.dtype != ref.dtype:
                 raise ValueError("qk_rmsnorm_rope: q/k layouts differ")
@@ -232,7 +238,7 @@ def qk_rmsnorm_rope(q=None, k=None, gamma_q=None, gamma_k=None, bias_q=None, bia
         if coords.dtype != torch.int32 or not coords.is_contiguous() or coords.shape[0] != rows:
             raise ValueError("qk_rmsnorm_rope: coords must be contiguous int32 [rows, 1+pos_dim]")
         cc = coords.shape[1]
-    p = lambda t: t.data_ptr() if t is not None else None
+    p = _ptr
     call("t2h_qk_rmsnorm_rope", p(q), p(k), p(q_out), p(k_out), rows, in_stride, out_stride, h, d, dt,
          p(bias_q), p(bias_k), p(gamma_q), p(gamma_k), int(bool(use_rope)), fp, fd, int(pos_dim), p(phases),
          ph_rows, p(coords), cc, int(grid_res), _stream())
@@ -250,7 +256,7 @@ def qkv_bias_rmsnorm_rope(qkv, heads: int, head_dim: int, bias=None, gamma_q=Non
     hold, fp, fd = _host_freqs(freqs if freqs is not None else [])
     ph_rows = phases.numel() // head_dim if phases is not None else 0
     cc = coords.shape[1] if coords is not None else 0
-    p = lambda t: t.data_ptr() if t is not None else None
+    p = _ptr
     call("t2h_qkv_bias_rmsnorm_rope", qkv.data_ptr(), rows, heads, head_dim, dt, p(bias), p(gamma_q), p(gamma_k),
          int(bool(use_rope)), fp, fd, int(pos_dim), p(phases), ph_rows, p(coords), cc, int(grid_res), _stream())
     del hold
@@ -270,7 +276,7 @@ def attn_pack(q=None, k=None, v=None, mp: int = 0, lp: int = 0, bias_q=None, bia
     rows, h, d, in_stride = _heads_view(ref, "attn_pack")
     dt = _dtype(ref, "attn_pack")
     for t in (q, k, v):
-        if t is not None:
+        if t is not None and t is not ref:
             if _heads_view(t, "attn_pack") != (rows, h, d, in_stride) or t.dtype != ref.dtype:
                 raise ValueError("attn_pack: q/k/v layouts differ")
     for g in (gamma_q, gamma_k, bias_q, bias_k, bias_v):
@@ -297,7 +303,7 @@ def attn_pack(q=None, k=None, v=None, mp: int = 0, lp: int = 0, bias_q=None, bia
         if coords.dtype != torch.int32 or not coords.is_contiguous() or coords.shape[0] != rows:
             raise ValueError("attn_pack: coords must be contiguous int32 [rows, 1+pos_dim]")
         cc = coords.shape[1]
-    p = lambda t: t.data_ptr() if t is not None else None
+    p = _ptr
     call("t2h_attn_pack", p(q), p(k), p(v), in_stride, rows, h, d, dt, p(bias_q), p(bias_k), p(bias_v), p(gamma_q),
          p(gamma_k), int(bool(use_rope)), fp, fd, int(pos_dim), p(phases), ph_rows, p(coords), cc, int(grid_res),
          p(qh), mp, p(ko), p(vh), lp, int(bool(k_transposed)), _stream())
@@ -331,7 +337,8 @@ def qkv_linear_pack(x, weight, heads: int, bias=None, gamma_q=None, gamma_k=None
         _dev(bias, "qkv_linear_pack")
         if bias.dtype != torch.float32 or bias.numel() != n or not bias.is_contiguous():
             raise ValueError("qkv_linear_pack: bias must be a contiguous float32 [3*H*D] tensor")
-        bq, bk, bv = bias.reshape(3, heads * d).unbind(0)
+        bq = bias.data_ptr()
+        bk, bv = bq + 4 * heads * d, bq + 8 * heads * d
     for g in (gamma_q, gamma_k):
         if g is not None:
             _dev(g, "qkv_linear_pack")
@@ -356,8 +363,8 @@ def qkv_linear_pack(x, weight, heads: int, bias=None, gamma_q=None, gamma_k=None
         if coords.dtype != torch.int32 or not coords.is_contiguous() or coords.shape[0] != rows:
             raise ValueError("qkv_linear_pack: coords must be contiguous int32 [rows, 1+pos_dim]")
         cc = coords.shape[1]
-    p = lambda t: t.data_ptr() if t is not None else None
-    call("t2h_qkv_linear_pack", x.data_ptr(), ldx, weight.data_ptr(), rows, k, heads, d, dt, p(bq), p(bk), p(bv),
+    p = _ptr
+    call("t2h_qkv_linear_pack", x.data_ptr(), ldx, weight.data_ptr(), rows, k, heads, d, dt, bq, bk, bv,
          p(gamma_q), p(gamma_k), int(bool(use_rope)), fp, fd, int(pos_dim), p(phases), ph_rows, p(coords), cc,
          int(grid_res), qh.data_ptr(), mp, ko.data_ptr(), vh.data_ptr(), lp, int(bool(k_transposed)), _stream())
     del hold
@@ -379,7 +386,7 @@ def rope_phases(rows: int, head_dim: int, freqs, pos_dim: int = 3, positions=Non
     if positions is not None and (positions.dtype != torch.float32 or not positions.is_contiguous()):
         raise ValueError("rope_phases: positions must be contiguous float32")
     cc = coords.shape[1] if coords is not None else 0
-    p = lambda t: t.data_ptr() if t is not None else None
+    p = _ptr
     call("t2h_rope_phases", out.data_ptr(), rows, head_dim, fp, fd, int(pos_dim), p(positions), p(coords), cc,
          int(grid_res), _stream())
     del hold
@@ -561,10 +568,10 @@ def flow_euler_step(x_t, v_pos, t: float, t_prev: float, sigma_min: float, v_neg
     rescale = v_neg is not None and guidance_strength not in (0.0, 1.0) and guidance_rescale > 0.0
     if rescale and ws is None:
         ws = torch.empty(flow_euler_workspace(rows, rs, nso), dtype=torch.uint8, device=x_t.device)
-    p = lambda t: t.data_ptr() if t is not None else None
+    p = _ptr
     call("t2h_flow_euler_step", x_t.data_ptr(), v_pos.data_ptr(), p(v_neg), x_prev.data_ptr(), p(x0), rows, rs, dt,
          float(t), float(t_prev), float(sigma_min), float(guidance_strength), float(guidance_rescale),
-         so.ctypes.data if so is not None else None, nso, p(ws), ws.numel() if ws is not None else 0, _stream())
+         so.__array_interface__["data"][0] if so is not None else None, nso, p(ws), ws.numel() if ws is not None else 0, _stream())
     return x_prev, x0
 
 

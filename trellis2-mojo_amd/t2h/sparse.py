@@ -234,7 +234,7 @@ class Modulation:
             m = self.lin(ops.activation(mod, ops.ACT_SILU)).to(torch.float32).contiguous()
         if m.dim() != 2 or m.shape[1] != 6 * channels:
             raise ValueError("Modulation: expected [N, 6C] modulation rows")
-        return [m[:, i * channels:(i + 1) * channels] for i in range(6)]
+        return [m.narrow(1, i * channels, channels) for i in range(6)]
 
 
 class SparseRotaryPositionEmbedder:
