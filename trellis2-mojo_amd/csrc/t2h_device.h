@@ -162,11 +162,12 @@ template <> __device__ __forceinline__ float ld1<__bf16>(const __bf16* p) {
 // gated-residual thread's eight) uses the default cache policy instead:
 // LN + modulate 201 -> 188 us, the config-5 chain 1,628 -> 1,601 us. All
 // non-temporal, or all cached, is slower. Launches that move less than
-// T2H_CACHED_SHARE_MIN bytes keep every load non-temporal: streams that fit
-// the 256 MB infinity cache read slower with the share when the cache holds
-// other dirty data.
+// T2H_CACHED_SHARE_MIN bytes keep every load non-temporal. The line from 512
+// to 100 MB: a block's glue (LN, two joins, residual) over 39,804 f16 rows 277
+// -> 265 us, 20,000 150.5 -> 146, 9,000 f32 rows 140 -> 137; launches below
+// 100 MB were the same with and without.
 #ifndef T2H_CACHED_SHARE_MIN
-#define T2H_CACHED_SHARE_MIN (int64_t(512) << 20)
+#define T2H_CACHED_SHARE_MIN (int64_t(100) << 20)
 #endif
 
 // E elements of T (E * sizeof(T) == 16) at element `off` of a wave-uniform
