@@ -268,3 +268,20 @@ def test_reference_attention_shapes(dev, rows, h):
         assert_close(qh, wq, torch.float32, f"qh rows={rows} h={h}")
         assert_close(ko if kt else ko.transpose(1, 2), wk, torch.float32, f"k transposed={kt} rows={rows} h={h}")
         assert np.array_equal(host(vh), wv), "v: bias add and pack are exact"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("rows, lp", [(1, 8), (15, 16), (63, 64), (65, 72), (130, 200)])
+def test_k_transposed_tile_edges(dev, dtype, d, rows, lp):
+    """The 16-bit tile is transposed in registers, 16 tokens a wave: token
+    counts that end inside a wave, an 8-token piece or a tile, pads that end a
+    tile early, and an odd head count, each exactly the row-major layout."""
+    h = 3
+    k = to_dev(orc.randn(2900 + rows, (rows, h, d)), dev, dtype)
+    gk = to_dev(_params(h, d, 2901)[2], dev)
+    coords = torch.arange(4 * rows, device=dev, dtype=torch.int32).view(rows, 4) % 61
+    kw = dict(gamma_k=gk, freqs=nn.rope_freqs(d), coords=coords, mp=lp, lp=lp)
+    _, kt, _ = ops.attn_pack(None, k, None, k_transposed=True, **kw)
+    _, kn, _ = ops.attn_pack(None, k, None, k_transposed=False, **kw)
+    assert torch.equal(kt, kn.transpose(1, 2))

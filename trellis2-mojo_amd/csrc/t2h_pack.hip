@@ -21,9 +21,9 @@
 //   tensor and loops over a group of heads; a wave instruction covers 4 rows
 //   of one head, the rows' cos/sin stay in registers across the heads. The
 //   transposed k goes through LDS (f32: 64 x (D+1), odd row pitch,
-//   conflict-free column reads; 16-bit: the output bits in two 64 x (D+2)
-//   buffers, one per alternate head, so one barrier per head) and leaves as
-//   16-byte vectors along the token axis.
+//   conflict-free column reads; 16-bit: transposed in registers, 16-byte
+//   pieces in two tiles for alternate heads, so one LDS-only barrier per head)
+//   and leaves as 16-byte vectors along the token axis.
 // On MI355X the row-major k ([H, lp, D]) is the faster layout: its rows are
 // what an MFMA attention kernel reads as the K operand.
 //
@@ -94,8 +94,91 @@ struct PackOrder {
     int8_t which[3];
 };
 
-template <typename T, int D, bool KT>
-__global__ __launch_bounds__(kPackBlock) void pack_tile_kernel(PackArgs a, RopeSlots tab, PackOrder order) {
+// The 16-bit transposed tile: a row of 64 tokens (128 bytes) per element.
+// Chunk c (8 tokens, 16 bytes) of element e; E = elements per lane = D / 16.
+// Lanes m = 0..15 write elements E m + const: eight of them take distinct
+// chunk positions and the other eight rows of the other parity, so the 16
+// pieces lie in distinct banks; a read takes whole rows.
+constexpr int kTileRow = 2 * kPackRows;
+template <int E>
+__device__ __forceinline__ int tile_at(int e, int c) {
+    return (e ^ ((e / (8 * E)) & 1)) * kTileRow + ((c ^ ((e / E) & 7)) * 16);
+}
+
+__device__ __forceinline__ void swap16(uint32_t& a, uint32_t& b) {     // odd 16-lane rows of a, even ones of b
+    const auto w = __builtin_amdgcn_permlane16_swap(a, b, false, false);
+    a = (uint32_t)w[0];
+    b = (uint32_t)w[1];
+}
+__device__ __forceinline__ void swap32(uint32_t& a, uint32_t& b) {     // upper half of a, lower half of b
+    const auto w = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+    a = (uint32_t)w[0];
+    b = (uint32_t)w[1];
+}
+// Elements 2k (lo) and 2k + 1 (hi) of four tokens' words.
+__device__ __forceinline__ void zip4(const uint32_t (&t)[4], uint32_t* lo, uint32_t* hi) {
+    lo[0] = __builtin_amdgcn_perm(t[1], t[0], 0x05040100);
+    lo[1] = __builtin_amdgcn_perm(t[3], t[2], 0x05040100);
+    hi[0] = __builtin_amdgcn_perm(t[1], t[0], 0x07060302);
+    hi[1] = __builtin_amdgcn_perm(t[3], t[2], 0x07060302);
+}
+
+// A wave's 16 token rows of one head, transposed in registers: row group g of
+// lanes holds token 4 it + g, lane m elements E m .. E m + E - 1 as words
+// w[it][..]. Row swaps and half swaps leave each lane one word (two elements)
+// of 16 tokens (E = 8) or of 8 (E = 4), which go to the tile as 16-byte
+// pieces along the tokens: 4 (2) LDS writes and 4 (2) reads per lane and head
+// in place of 32 + 32 (16 + 16) 2-byte ones. With the choice of heads per
+// block below, k alone (12 x 128, f16): 9,000 rows 22.3 -> 19.6 us, 20,000
+// 43.4 -> 31.6, 39,804 59.7 -> 58.0, 150,000 199.7 -> 191.9 (4.8 TB/s); what
+// bounds the large ones is the 128-byte pieces of the strided output planes.
+template <int E>
+__device__ __forceinline__ void transpose_to_tile(uint32_t (&w)[kPackIters][E / 2], uint8_t* buf, int wave, int g,
+                                                  int m) {
+    static_assert(kPackIters == 4 && (E == 8 || E == 4), "16 tokens per wave");
+    uint32_t lo[8], hi[8];
+    if constexpr (E == 8) {
+#pragma unroll
+        for (int it = 0; it < 4; ++it) {
+            swap16(w[it][0], w[it][2]);      // rows 0, 2: word 0 of tokens g, g + 1; rows 1, 3: word 2
+            swap16(w[it][1], w[it][3]);
+            swap32(w[it][0], w[it][1]);      // lower half: words 0 and 2 of tokens 0, 2; upper: 1 and 3
+            swap32(w[it][2], w[it][3]);      // ... of tokens 1, 3
+            const uint32_t t[4] = {w[it][0], w[it][2], w[it][1], w[it][3]};
+            zip4(t, lo + 2 * it, hi + 2 * it);
+        }
+        const int e = E * m + 2 * (2 * (g & 1) + (g >> 1));
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            *reinterpret_cast<u32x4*>(buf + tile_at<E>(e, 2 * wave + q)) =
+                u32x4{lo[4 * q], lo[4 * q + 1], lo[4 * q + 2], lo[4 * q + 3]};
+            *reinterpret_cast<u32x4*>(buf + tile_at<E>(e + 1, 2 * wave + q)) =
+                u32x4{hi[4 * q], hi[4 * q + 1], hi[4 * q + 2], hi[4 * q + 3]};
+        }
+    } else {
+#pragma unroll
+        for (int it = 0; it < 4; ++it) swap16(w[it][0], w[it][1]);      // rows 0, 2: word 0; rows 1, 3: word 1
+#pragma unroll
+        for (int it = 0; it < 2; ++it) {     // lower half: tokens 4 it .. of the wave; upper: 8 + 4 it ..
+            swap32(w[it][0], w[it + 2][0]);
+            swap32(w[it][1], w[it + 2][1]);
+            const uint32_t t[4] = {w[it][0], w[it][1], w[it + 2][0], w[it + 2][1]};
+            zip4(t, lo + 2 * it, hi + 2 * it);
+        }
+        const int e = E * m + 2 * (g & 1), c = 2 * wave + (g >> 1);
+        *reinterpret_cast<u32x4*>(buf + tile_at<E>(e, c)) = u32x4{lo[0], lo[1], lo[2], lo[3]};
+        *reinterpret_cast<u32x4*>(buf + tile_at<E>(e + 1, c)) = u32x4{hi[0], hi[1], hi[2], hi[3]};
+    }
+}
+
+// AHEAD (16-bit transposed k, blocks of several heads): the first head's rows
+// are requested between the positions' loads and the phases (39,804 x 12 x
+// 128: 60.9 -> 58.0 us), in 128 registers for 4 waves per SIMD. Blocks of one
+// head, in launches that are resident at once anyway, fetch after the phases
+// and keep their registers (2,369 rows: 9.8 against 10.4 us). Rows ahead of
+// the positions make the phases wait for them (62.8 us).
+template <typename T, int D, bool KT, bool AHEAD>
+__global__ __launch_bounds__(kPackBlock, AHEAD ? 4 : 1) void pack_tile_kernel(PackArgs a, RopeSlots tab, PackOrder order) {
     using L = HeadLanes<T, D>;
     constexpr int E = L::E;
     constexpr int P = L::P;
@@ -104,7 +187,7 @@ __global__ __launch_bounds__(kPackBlock) void pack_tile_kernel(PackArgs a, RopeS
     // is written while the previous head's is read (one barrier per head).
     constexpr bool kTwo = KT && sizeof(T) == 2;
     __shared__ float tile[KT && !kTwo ? kPackRows : 1][KT && !kTwo ? D + 1 : 1];
-    __shared__ uint16_t tile2[kTwo ? 2 : 1][kTwo ? kPackRows : 1][kTwo ? D + 2 : 1];
+    __shared__ __attribute__((aligned(16))) uint8_t tile2[kTwo ? 2 : 1][kTwo ? D * kTileRow : 16];
     const int lane = lane_id();
     const int g = lane >> 4;
     const int m = lane & 15;
@@ -123,13 +206,32 @@ __global__ __launch_bounds__(kPackBlock) void pack_tile_kernel(PackArgs a, RopeS
     // with no token rows every output is a pad: no phase (coords) or row read
     const bool rope = a.use_rope && which < 2 && a.rows > 0;
 
-    // this lane's token rows (clamped for the loads; rows >= a.rows are pads)
+    // this lane's token rows (clamped for the loads; rows >= a.rows are pads);
+    // the register transpose wants a wave's 16 rows consecutive
+    const auto row_of = [&](int it) {
+        return kTwo ? wave * (4 * kPackIters) + it * 4 + g : it * kPackRowsPerIter + wave * 4 + g;
+    };
     int64_t rl[kPackIters];
 #pragma unroll
     for (int it = 0; it < kPackIters; ++it) {
-        const int64_t t = t0 + it * kPackRowsPerIter + wave * 4 + g;
+        const int64_t t = t0 + row_of(it);
         rl[it] = t < a.rows ? t : (a.rows > 0 ? a.rows - 1 : 0);
     }
+
+    // The transposed path fetches head z + 1 (rows and the head's bias and
+    // gamma) before it stores head z, so a block's loads overlap its own
+    // stores and no parameter load waits for them (loads and stores share
+    // vmcnt on gfx9).
+    RawRow<T, D> raw[kPackIters];
+    float bv[E], gv[E];
+    auto fetch = [&](int z) {
+        if (a.rows > 0) {
+#pragma unroll
+            for (int it = 0; it < kPackIters; ++it) raw[it].load(in + rl[it] * a.in_stride + (int64_t)z * D, m);
+        }
+        if (bias != nullptr) L::params(bias + z * D, m, bv);
+        if (gamma != nullptr) L::params(gamma + z * D, m, gv);
+    };
 
     // cos/sin of this lane's P slots for each of its rows, shared by all heads
     float pc[kPackIters][P], ps[kPackIters][P];
@@ -149,31 +251,31 @@ __global__ __launch_bounds__(kPackBlock) void pack_tile_kernel(PackArgs a, RopeS
                 ax[j] = tab.axis[L::slot(m, j)];
                 fr[j] = tab.freq[L::slot(m, j)];
             }
+            if constexpr (AHEAD) {
+                float pos[kPackIters][T2H_MAX_POS_DIM];
 #pragma unroll
-            for (int it = 0; it < kPackIters; ++it) {
-                float pos[T2H_MAX_POS_DIM];
-                src.get(rl[it], pos);
+                for (int it = 0; it < kPackIters; ++it) src.get(rl[it], pos[it]);
+                fetch(hg * order.hpb);
+                __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int j = 0; j < P; ++j) slot_phase(pos, ax[j], fr[j], pc[it][j], ps[it][j]);
+                for (int it = 0; it < kPackIters; ++it)
+#pragma unroll
+                    for (int j = 0; j < P; ++j) slot_phase(pos[it], ax[j], fr[j], pc[it][j], ps[it][j]);
+            } else {
+#pragma unroll
+                for (int it = 0; it < kPackIters; ++it) {
+                    float pos[T2H_MAX_POS_DIM];
+                    src.get(rl[it], pos);
+#pragma unroll
+                    for (int j = 0; j < P; ++j) slot_phase(pos, ax[j], fr[j], pc[it][j], ps[it][j]);
+                }
             }
         }
     }
+    if constexpr (KT) {
+        if (!AHEAD || !rope || a.phases != nullptr) fetch(hg * order.hpb);
+    }
 
-    // The transposed path fetches head z + 1 (rows and the head's bias and
-    // gamma) before it stores head z, so a block's loads overlap its own
-    // stores and no parameter load waits for them (loads and stores share
-    // vmcnt on gfx9).
-    RawRow<T, D> raw[kPackIters];
-    float bv[E], gv[E];
-    auto fetch = [&](int z) {
-        if (a.rows > 0) {
-#pragma unroll
-            for (int it = 0; it < kPackIters; ++it) raw[it].load(in + rl[it] * a.in_stride + (int64_t)z * D, m);
-        }
-        if (bias != nullptr) L::params(bias + z * D, m, bv);
-        if (gamma != nullptr) L::params(gamma + z * D, m, gv);
-    };
-    if constexpr (KT) fetch(hg * order.hpb);
     for (int zi = 0; zi < order.hpb; ++zi) {
         const int z = hg * order.hpb + zi;
         if constexpr (!KT) fetch(z);
@@ -192,9 +294,10 @@ __global__ __launch_bounds__(kPackBlock) void pack_tile_kernel(PackArgs a, RopeS
 #pragma unroll
             for (int i = 0; i < E; ++i) gsc[i] = gv[i] * a.rms_scale;
         }
+        uint32_t pw[kTwo ? kPackIters : 1][E / 2];
 #pragma unroll
         for (int it = 0; it < kPackIters; ++it) {
-            const int64_t t = t0 + it * kPackRowsPerIter + wave * 4 + g;
+            const int64_t t = t0 + row_of(it);
             float* x = v[it];
             if (bias != nullptr) {
 #pragma unroll
@@ -219,16 +322,10 @@ __global__ __launch_bounds__(kPackBlock) void pack_tile_kernel(PackArgs a, RopeS
                 for (int i = 0; i < E; ++i) x[i] = 0.0f;
             }
             if constexpr (kTwo) {
-                // elements 2i, 2i+1 of a lane are adjacent (pieces of >= 2 elements)
-                const int tl = it * kPackRowsPerIter + wave * 4 + g;
 #pragma unroll
-                for (int i = 0; i < E; i += 2) {
-                    const uint32_t w = Word<T>::pack(x + i);
-                    tile2[zi & 1][tl][L::elem(m, i)] = (uint16_t)w;
-                    tile2[zi & 1][tl][L::elem(m, i) + 1] = (uint16_t)(w >> 16);
-                }
+                for (int i = 0; i < E / 2; ++i) pw[it][i] = Word<T>::pack(x + 2 * i);
             } else if constexpr (KT) {
-                const int tl = it * kPackRowsPerIter + wave * 4 + g;
+                const int tl = row_of(it);
 #pragma unroll
                 for (int i = 0; i < E; ++i) tile[tl][L::elem(m, i)] = round_to<T>(x[i]);
             } else if (t < extent) {
@@ -236,22 +333,22 @@ __global__ __launch_bounds__(kPackBlock) void pack_tile_kernel(PackArgs a, RopeS
             }
         }
         if constexpr (kTwo) {
+            uint8_t* buf = tile2[zi & 1];
+            transpose_to_tile<E>(pw, buf, wave, g, m);
             // this head's tile is whole, and every read of the tile written
-            // two heads ago (the other buffer's previous contents) is done
-            __syncthreads();
+            // two heads ago (the other buffer's previous contents) is done.
+            // Only LDS is shared: the previous head's stores stay in flight
+            lds_barrier();
             if (zi + 1 < order.hpb) fetch(z + 1);
             constexpr int VE = kPack<T>;
             constexpr int VPR = kPackRows / VE;
+#pragma unroll AHEAD ? 1 : D * VPR / kPackBlock
             for (int vi = threadIdx.x; vi < D * VPR; vi += kPackBlock) {
                 const int e = vi / VPR;
-                const int tq = (vi % VPR) * VE;
-                if (t0 + tq >= extent) continue;
-                uint16_t w[VE];
-#pragma unroll
-                for (int i = 0; i < VE; ++i) w[i] = tile2[zi & 1][tq + i][e];
-                u32x4 o;
-                __builtin_memcpy(&o, w, 16);
-                u32x4* dst = reinterpret_cast<u32x4*>(out + ((int64_t)z * D + e) * a.lp + t0 + tq);
+                const int c = vi % VPR;
+                if (t0 + c * VE >= extent) continue;
+                const u32x4 o = *reinterpret_cast<const u32x4*>(buf + tile_at<E>(e, c));
+                u32x4* dst = reinterpret_cast<u32x4*>(out + ((int64_t)z * D + e) * a.lp + t0 + c * VE);
                 if (T2H_NT) __builtin_nontemporal_store(o, dst); else *dst = o;
             }
         } else if constexpr (KT) {
@@ -565,6 +662,30 @@ int heads_per_block(int64_t tiles, int tensors, int heads) {
     return best;
 }
 
+// The same for the 16-bit transposed k: the least modelled time, rounds of
+// resident blocks (4 per CU, 6 for head_dim 64, one less without AHEAD: registers) times a block's
+// fixed part (16 or 8 sincosf per lane, first loads) and its heads. us by
+// heads per block, 12 heads of 128: 9,000 rows 22.8 (1), 19.4 (2), 20.8 (4),
+// 24.2 (6), 35.7 (12); 39,804 rows 80.7, 63.4 (2), 61.5 (3), 58.2 (4), 64.7
+// (6), 56.6 (12); 120,000 rows 228, 172 (2), 158 (4), 155 (6), 154 (12). 16
+// heads of 64: 39,804 rows 41.9 (4), 38.3 (8), 44.9 (16); 100,000 rows 107
+// (4), 94.6 (8), 104 (16).
+int heads_per_block_kt(int64_t tiles, int heads, int head_dim) {
+    int best = 1;
+    int64_t least = 0;
+    for (int hpb = 1; hpb <= heads; ++hpb) {
+        if (heads % hpb) continue;
+        const int64_t resident = ((head_dim == 64 ? 6LL : 4LL) - (hpb == 1)) * device_cu_count();
+        const int64_t rounds = (tiles * (heads / hpb) + resident - 1) / resident;
+        const int64_t cost = rounds * (3 + hpb);
+        if (least == 0 || cost < least) {
+            least = cost;
+            best = hpb;
+        }
+    }
+    return best;
+}
+
 template <typename T, int D>
 hipError_t launch_d(const PackArgs& a, const RopeSlots& tab, hipStream_t s) {
     const int64_t ext = a.mp > a.lp ? a.mp : a.lp;
@@ -590,7 +711,7 @@ hipError_t launch_d(const PackArgs& a, const RopeSlots& tab, hipStream_t s) {
         rows.hpb = heads_per_block(tiles, rows.n, a.heads);
         rows.groups = a.heads / rows.hpb;
         const int64_t blocks = tiles * rows.groups * rows.n;
-        hipLaunchKernelGGL((pack_tile_kernel<T, D, false>), grid_1d(blocks), dim3(kPackBlock), 0, s, a, tab,
+        hipLaunchKernelGGL((pack_tile_kernel<T, D, false, false>), grid_1d(blocks), dim3(kPackBlock), 0, s, a, tab,
                            rows);
         if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
     }
@@ -598,10 +719,12 @@ hipError_t launch_d(const PackArgs& a, const RopeSlots& tab, hipStream_t s) {
         PackOrder kt{};
         kt.n = 1;
         kt.which[0] = 1;
-        kt.hpb = heads_per_block(tiles, 1, a.heads);
+        kt.hpb = sizeof(T) == 2 ? heads_per_block_kt(tiles, a.heads, D) : heads_per_block(tiles, 1, a.heads);
         kt.groups = a.heads / kt.hpb;
-        hipLaunchKernelGGL((pack_tile_kernel<T, D, true>), grid_1d(tiles * kt.groups), dim3(kPackBlock), 0,
-                           s, a, tab, kt);
+        const dim3 grid = grid_1d(tiles * kt.groups);
+        if (sizeof(T) == 2 && kt.hpb > 1)
+            hipLaunchKernelGGL((pack_tile_kernel<T, D, true, sizeof(T) == 2>), grid, dim3(kPackBlock), 0, s, a, tab, kt);
+        else hipLaunchKernelGGL((pack_tile_kernel<T, D, true, false>), grid, dim3(kPackBlock), 0, s, a, tab, kt);
         return hipGetLastError();
     }
     return hipSuccess;
