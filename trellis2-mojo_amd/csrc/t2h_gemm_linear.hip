@@ -376,6 +376,8 @@ __global__ __launch_bounds__(64 * WF * WT, 1) void gemm_small_kernel(GemmArgs a)
         step(af[1], bf[1], af[0], bf[0], s + 1);
     }
     if (s < nst) step(af[0], bf[0], af[1], bf[1], s);
+    // the loads issued past the last stage land in LDS that only this block
+    // owns, and a wave's end waits for its outstanding memory operations
 
     const BatchMap bm{a.batch.offsets, a.batch.rows_per_batch, a.batch.nbatch};
     const bool has_bias = a.bias != nullptr, has_gate = RES && a.gate != nullptr;
