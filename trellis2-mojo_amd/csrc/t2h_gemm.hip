@@ -22,9 +22,13 @@ namespace {
 // cos/sin from positions: computing them per head and token (64 sincosf per
 // token and head) took 395 us of the 3,243 us of 201,436 tokens x 4608
 // features. Voxel coordinates are small integers, so each block computes
-// cos/sin of every (position < kPos, frequency) once, into LDS, with the same
-// sincosf of the same f32 angle, and its tiles look them up; a token outside
-// the table takes the direct computation.
+// cos/sin of every (position, frequency) once, into LDS, with the same sincosf
+// of the same f32 angle, and its tiles look them up: the first 161 positions
+// for 21 frequencies (heads of 128, three axes), 256 for 10 (heads of 64). 16
+// tokens of which one lies outside are computed, from the positions and
+// frequencies in LDS. us, all inside / all outside / no table (f16, bias, RMS):
+// heads of 128, 2,369 tokens 48 / 56 / 61, 39,804 529 / 590 / 654, 201,436
+// 2,690 / 2,930 / 3,250; heads of 64, 39,804 255 / 275 / 344.
 //
 // The values leave as whole 128-byte row pieces: through 2 KB of LDS per wave
 // (16 tokens x 64 features) for qh [H, mp, D], k [H, lp, D], vh [H, lp, D];
@@ -33,18 +37,29 @@ namespace {
 // the next tile's operands only afterwards). Tiles past the last token row
 // skip the GEMM and write the pads.
 constexpr int kHead = 128;                     // features of a wave
-constexpr int kPos = 128;                      // positions of the cos/sin table, where they fit
-// LDS past the stages: [wave half][bias, gamma * sqrt(D)][128] f32, the tile's
-// packed positions, the slots' table columns, the table
-constexpr int kPosOff = 2048, kSlotOff = kPosOff + 1024, kTabOff = kSlotOff + 256, kExtra = 32768;
-constexpr int kTabEntries = (kExtra - kTabOff) / 8;
-constexpr uint32_t kNoPos = 0xFFFFFFFFu;       // a token whose position is not in the table
+constexpr int kPos = 256;                      // most positions of the cos/sin table
+// LDS past the stages: [wave half][bias, gamma * sqrt(D)][128] f32, the slots'
+// table columns and frequencies, the tile's positions ([axes 0, 2 | axes 1,
+// 3][256], two 16-bit halves a word), the table
+constexpr int kSlotOff = 2048, kFreqOff = kSlotOff + 256, kPosOff = kFreqOff + 256, kExtra = 32768;
+static_assert(T2H_MAX_POS_DIM == 4, "two words of two axes");
+constexpr int kFar = -32768;                   // lower half: a coordinate past 16 bits, read again where needed
 
 // Slot of a 16-byte chunk in a staged 256-byte token row: chunk c of row r
 // at c ^ stage_swz(r). Over 16 consecutive rows (one write) every slot appears
 // once; over rows 8g + j, g = 0..7 (one transposed gather) the slots are
 // distinct; a row's 16 chunks are a permutation.
 __device__ __forceinline__ int stage_swz(int r) { return ((r >> 3) ^ ((r & 7) << 1)) & 15; }
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// A launch parameter as a value of its own: a divisor's reciprocal or a flag
+// derived from it would be computed ahead of the tile loop and sit, or be
+// spilled, in registers that the loop needs.
+template <typename V> __device__ __forceinline__ V fresh(V d) {
+    asm volatile("" : "+s"(d));
+    return d;
+}
 
 template <typename T, bool KT, int HD, int BT, bool W64>
 __global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackArgs p, RopeSlots tab) {
@@ -64,7 +79,9 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackA
     const float* pg = reinterpret_cast<const float*>(extra) + (wf * 2 + 1) * kHead;
     const bool lookup = p.use_rope && p.phases == nullptr && g.rows > 0;
     const int fd = p.freq_dim;
-    const int npos = fd > 0 ? (kTabEntries - 1) / fd < kPos ? (kTabEntries - 1) / fd : kPos : 0;
+    const int tab_off = kPosOff + (p.pos_dim > 1 ? 2048 : 1024);
+    const int fit = fd > 0 ? ((kExtra - tab_off) / 8 - 1) / fd : 0;
+    const int npos = fit < kPos ? fit : kPos;
 
     int64_t tt, ft;
     tile_at(g, walk.lo + walk.i, tt, ft);
@@ -75,18 +92,28 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackA
     if (lookup) {
         // entry pos * fd + f: (cos, sin); the last entry is the identity. A
         // slot's word: its column's byte offset | axis << 16 (4: none)
-        float2* t = reinterpret_cast<float2*>(extra + kTabOff);
-        for (int e = threadIdx.x; e < npos * fd; e += kThreads) {
-            const float pos = (float)(e / fd);
-            float cv, sv;
-            slot_phase(&pos, 0, tab.freq[e % fd], cv, sv);
-            t[e] = float2{cv, sv};
-        }
-        if (threadIdx.x == 0) t[npos * fd] = float2{1.0f, 0.0f};
+        const float* freqs = reinterpret_cast<const float*>(extra + kFreqOff);
+        float2* t = reinterpret_cast<float2*>(extra + tab_off);
         if (threadIdx.x < HD / 2) {
             const int ax = slot_axis(threadIdx.x, fd, p.pos_dim);
             reinterpret_cast<uint32_t*>(extra + kSlotOff)[threadIdx.x] =
                 ax < 0 ? (uint32_t)(npos * fd * 8) | (4u << 16) : (uint32_t)((threadIdx.x - ax * fd) * 8) | (ax << 16);
+            reinterpret_cast<float*>(extra + kFreqOff)[threadIdx.x] = tab.freq[threadIdx.x];
+        }
+        if (threadIdx.x == 0) t[npos * fd] = float2{1.0f, 0.0f};
+        wait_lds();
+        turn_barrier();
+        if (fd > 0) {
+            int pos = threadIdx.x / fd, f = threadIdx.x - pos * fd;
+            const int dp = kThreads / fd, df = kThreads - dp * fd;
+            while (pos < npos) {
+                const float x = (float)pos;
+                float cv, sv;
+                slot_phase(&x, 0, freqs[f], cv, sv);
+                t[pos * fd + f] = float2{cv, sv};
+                pos += dp + (f + df >= fd);
+                f += df - (f + df >= fd ? fd : 0);
+            }
         }
         wait_lds();
     }
@@ -98,7 +125,7 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackA
         const float* __restrict__ bias = which == 0 ? p.bias_q : which == 1 ? p.bias_k : p.bias_v;
         const float* __restrict__ gamma = which == 0 ? p.gamma_q : which == 1 ? p.gamma_k : nullptr;
         const bool rope = p.use_rope && which < 2 && g.rows > 0;
-        // one bias or gamma value and one token's position per thread, read
+        // one bias or gamma value and one word of positions per thread, read
         // ahead of the main loop and staged in LDS after it
         float pv;
         {
@@ -107,20 +134,19 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackA
             pv = src != nullptr ? src[f] : 0.0f;
             if ((i >> 7) & 1) pv *= p.rms_scale;
         }
-        uint32_t pw = kNoPos;
-        if (rope && lookup && threadIdx.x < BT) {
-            const int64_t t = t0 + threadIdx.x < g.rows ? t0 + threadIdx.x : g.rows - 1;
-            const PosSource src{p.coords, p.coord_cols, p.grid_res, p.pos_dim};
-            float pos[T2H_MAX_POS_DIM];
-            src.get(t, pos);
-            bool in = true;
-            uint32_t w = 0;
-#pragma unroll
-            for (int ax = 0; ax < T2H_MAX_POS_DIM; ++ax) {
-                in = in && pos[ax] >= 0.0f && pos[ax] < (float)npos;
-                w |= ((uint32_t)(int)pos[ax] & 0xFFu) << (8 * ax);
+        const int pax = wave / (BT / 64);       // axes pax and pax + 2, or (0) the phase table's row
+        const bool has_pos = rope && pax < (lookup ? p.pos_dim < 2 ? 1 : 2 : 1);
+        uint32_t pw = 0;
+        if (has_pos) {
+            const int64_t t = t0 + threadIdx.x % BT, tc = t < g.rows ? t : g.rows - 1;
+            if (!lookup) {
+                pw = (uint32_t)(tc % fresh(p.phase_rows));
+            } else {
+                const PosSource src{fresh(p.coords), p.coord_cols, fresh(p.grid_res), p.pos_dim};
+                const int lo = src.at(tc, pax), hi = pax + 2 < fresh(p.pos_dim) ? src.at(tc, pax + 2) : 0;
+                const bool near = lo == (int16_t)lo && hi == (int16_t)hi && lo != kFar;
+                pw = near ? (uint32_t)(uint16_t)lo | (uint32_t)hi << 16 : (uint32_t)(uint16_t)kFar;
             }
-            pw = in ? w : kNoPos;
         }
         f32x4 acc[8][kTJ];
         if (t0 < g.rows) {
@@ -144,7 +170,7 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackA
             if (!trans) c.prologue(steps);
         }
         reinterpret_cast<float*>(extra)[threadIdx.x] = pv;
-        if (threadIdx.x < BT) reinterpret_cast<uint32_t*>(extra + kPosOff)[threadIdx.x] = pw;
+        if (has_pos) reinterpret_cast<uint32_t*>(extra + kPosOff)[pax * 256 + threadIdx.x % BT] = pw;
         wait_lds();
         turn_barrier();
 
@@ -193,52 +219,65 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackA
             const int64_t t = tw + j * 16 + fr;
             const int64_t tc = t < g.rows ? t : g.rows - 1;   // clamped for position reads
             const bool live = t < g.rows;
-            uint32_t pos = kNoPos;
-            if (rope && lookup) pos = reinterpret_cast<const uint32_t*>(extra + kPosOff)[wt * Big<BT>::kWT + j * 16 + fr];
-            const bool direct = rope && lookup && __any(pos == kNoPos);
+            f32x16 cs;
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf) {
-                // cos/sin of the lane's slot pairs: cs[i] = (c, s) of slots s0 + i * 8, + 1
+                // cos/sin of the lane's slot pairs: cs[4 i ..] = (c, s) of slots s0 + i * 8, + 1
+                // (both halves are whole heads of 64: the same slots)
                 const int s0 = (FPH == 8 ? hf * 32 : 0) + h * 2;
-                f32x4 cs[4];
-                if (rope) {
+                if (rope && (FPH == 8 || hf == 0)) {
+                    const uint32_t* words = reinterpret_cast<const uint32_t*>(extra + kPosOff);
+                    const uint32_t w0 = words[wt * Big<BT>::kWT + j * 16 + fr];
                     if (!lookup) {
-                        const float* row = p.phases + (tc % p.phase_rows) * HD + s0 * 2;
-#pragma unroll
-                        for (int i = 0; i < 4; ++i) cs[i] = *reinterpret_cast<const f32x4*>(row + i * 16);
-                    } else if (!direct) {
-                        const uint32_t rowb = (uint32_t)fd * 8;
-                        const uint32_t r0 = (pos & 255) * rowb, r1 = ((pos >> 8) & 255) * rowb,
-                                       r2 = ((pos >> 16) & 255) * rowb, r3 = (pos >> 24) * rowb;
+                        const float* row = p.phases + (int64_t)w0 * HD + s0 * 2;
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
-                            const u32x2 sw = *reinterpret_cast<const u32x2*>(extra + kSlotOff + (s0 + i * 8) * 4);
+                            const f32x4 v = *reinterpret_cast<const f32x4*>(row + i * 16);
 #pragma unroll
-                            for (int q = 0; q < 2; ++q) {
-                                const uint32_t ax = sw[q] >> 16;
-                                const uint32_t ro = ax == 0 ? r0 : ax == 1 ? r1 : ax == 2 ? r2 : ax == 3 ? r3 : 0u;
-                                const float2 v =
-                                    *reinterpret_cast<const float2*>(extra + kTabOff + ro + (sw[q] & 0xFFFFu));
-                                cs[i][2 * q] = v.x;
-                                cs[i][2 * q + 1] = v.y;
-                            }
+                            for (int e = 0; e < 4; ++e) cs[i * 4 + e] = v[e];
                         }
                     } else {
-                        const PosSource src{p.coords, p.coord_cols, p.grid_res, p.pos_dim};
-                        float ps[T2H_MAX_POS_DIM];
-                        src.get(tc, ps);
-                        // rolled: unrolled, its sincosf calls crowd the registers of the path that is taken
-#pragma unroll 1
-                        for (int sl = 0; sl < 8; ++sl) {
-                            const int slot = s0 + (sl >> 1) * 8 + (sl & 1);
-                            float cv, sv;
-                            slot_phase(ps, tab.axis[slot], tab.freq[slot], cv, sv);
+                        const uint32_t w1 = p.pos_dim > 1 ? words[256 + wt * Big<BT>::kWT + j * 16 + fr] : 0;
+                        const int co[4] = {(int16_t)w0, (int16_t)w1, (int)w0 >> 16, (int)w1 >> 16};
+                        bool in = true;
 #pragma unroll
-                            for (int m = 0; m < 8; ++m)
-                                if (m == sl) {
-                                    cs[m >> 1][2 * (m & 1)] = cv;
-                                    cs[m >> 1][2 * (m & 1) + 1] = sv;
+                        for (int ax = 0; ax < 4; ++ax) in = in && (uint32_t)co[ax] < (uint32_t)npos;
+                        if (__all(in)) {
+                            const uint32_t rowb = (uint32_t)fd * 8;
+                            const uint32_t r0 = co[0] * rowb, r1 = co[1] * rowb, r2 = co[2] * rowb, r3 = co[3] * rowb;
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const u32x2 sw = *reinterpret_cast<const u32x2*>(extra + kSlotOff + (s0 + i * 8) * 4);
+#pragma unroll
+                                for (int q = 0; q < 2; ++q) {
+                                    const uint32_t ax = sw[q] >> 16;
+                                    const uint32_t ro = ax == 0 ? r0 : ax == 1 ? r1 : ax == 2 ? r2 : ax == 3 ? r3 : 0u;
+                                    const float2 v =
+                                        *reinterpret_cast<const float2*>(extra + tab_off + ro + (sw[q] & 0xFFFFu));
+                                    cs[i * 4 + q * 2] = v.x;
+                                    cs[i * 4 + q * 2 + 1] = v.y;
                                 }
+                            }
+                        } else {
+                            float pos[T2H_MAX_POS_DIM] = {(float)co[0], (float)co[1], (float)co[2], (float)co[3]};
+                            if (co[0] == kFar || co[1] == kFar) {
+                                PosSource{fresh(p.coords), p.coord_cols, fresh(p.grid_res), p.pos_dim}.get(tc, pos);
+                                // waited for here: at its use, every token would wait for the stores in flight
+#pragma unroll
+                                for (int ax = 0; ax < T2H_MAX_POS_DIM; ++ax) asm volatile("" : "+v"(pos[ax]));
+                            }
+                            // rolled: unrolled, its sincosf calls crowd the registers of the path that is taken
+#pragma unroll 1
+                            for (int n = 0; n < 8; ++n) {
+                                const int at = (s0 + (n >> 1) * 8 + (n & 1)) * 4;
+                                const uint32_t ax = *reinterpret_cast<const uint32_t*>(extra + kSlotOff + at) >> 16;
+                                const float fq = *reinterpret_cast<const float*>(extra + kFreqOff + at);
+                                const float lo = ax & 1 ? pos[1] : pos[0], hi = ax & 1 ? pos[3] : pos[2];
+                                float cv, sv;
+                                sincosf(mul_rn(ax & 2 ? hi : lo, fq), &sv, &cv);
+                                cs[2 * n] = ax & 4 ? 1.0f : cv;
+                                cs[2 * n + 1] = ax & 4 ? 0.0f : sv;
+                            }
                         }
                     }
                 }
@@ -248,8 +287,8 @@ __global__ __launch_bounds__(kThreads, 1) void qkv_pack_kernel(GemmArgs g, PackA
 #pragma unroll
                     for (int e = 0; e < 4; ++e) v[e] = acc[hf * 4 + i][j][e];
                     if (rope) {
-                        rotate_pair(v[0], v[1], cs[i][0], cs[i][1]);
-                        rotate_pair(v[2], v[3], cs[i][2], cs[i][3]);
+                        rotate_pair(v[0], v[1], cs[i * 4], cs[i * 4 + 1]);
+                        rotate_pair(v[2], v[3], cs[i * 4 + 2], cs[i * 4 + 3]);
                     }
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {

@@ -29,6 +29,12 @@ struct PosSource {
             pos[3] = 0.0f;
         }
     }
+    // the same along one axis (< pos_dim), as the integer it is
+    __device__ __forceinline__ int32_t at(int64_t r, int ax) const {
+        if (coords != nullptr) return coords[r * (int64_t)coord_cols + 1 + ax];
+        const int64_t R = grid_res;
+        return (int32_t)(r % (R * R * R) / (ax == 0 ? R * R : ax == 1 ? R : 1) % R);
+    }
 };
 
 // Axis of rotary slot p (< head_dim / 2): p / freq_dim for the pos_dim *
