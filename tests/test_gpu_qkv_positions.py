@@ -10,7 +10,7 @@ from t2h import nn, ops
 
 pytestmark = pytest.mark.gpu
 
-# around the table's ends (161 or 167 positions for 21 frequencies, 256 at
+# around the table's ends (167 positions for 21 frequencies, 256 at
 # most), around 16 bits, and the ends of int32
 ODD = np.array([-1, -77, 127, 128, 160, 161, 166, 167, 168, 255, 256, 5000, 32767, 32768, -32767, -32768, -32769,
                 1 << 24, (1 << 31) - 1, -(1 << 31)], np.int64).astype(np.int32)

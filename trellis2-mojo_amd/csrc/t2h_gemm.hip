@@ -23,7 +23,7 @@ namespace {
 // token and head) took 395 us of the 3,243 us of 201,436 tokens x 4608
 // features. Voxel coordinates are small integers, so each block computes
 // cos/sin of every (position, frequency) once, into LDS, with the same sincosf
-// of the same f32 angle, and its tiles look them up: the first 161 positions
+// of the same f32 angle, and its tiles look them up: the first 167 positions
 // for 21 frequencies (heads of 128, three axes), 256 for 10 (heads of 64). 16
 // tokens of which one lies outside are computed, from the positions and
 // frequencies in LDS. us, all inside / all outside / no table (f16, bias, RMS):
