@@ -101,8 +101,9 @@ def test_k_layouts_agree(dev, dtype, d):
 def test_k_transposed_head_groups(dev, dtype, rows):
     """The transposed-k tile kernel walks a group of heads per block, the
     16-bit tiles alternating between two LDS buffers from head to head. On
-    256 CUs these row counts give 2, 3, 6 and 12 heads per block; each must
-    equal the row-major layout (another kernel) exactly."""
+    256 CUs these row counts give 6, 4, 4 and 6 heads per block (the others:
+    test_k_transposed_every_head_group); each must equal the row-major layout
+    (another kernel) exactly."""
     h, d = 12, 128
     g = torch.Generator(device=dev).manual_seed(rows)
     qkv = torch.randn((rows, 3, h, d), generator=g, device=dev).to(dtype)
@@ -114,6 +115,38 @@ def test_k_transposed_head_groups(dev, dtype, rows):
     _, kt, _ = ops.attn_pack(None, qkv[:, 1], None, k_transposed=True, **kw)
     _, kn, _ = ops.attn_pack(None, qkv[:, 1], None, k_transposed=False, **kw)
     assert torch.equal(kt, kn.transpose(1, 2)), rows
+
+
+# (heads, head_dim, rows, heads per block on 256 CUs), none a whole tile of 64
+HEAD_GROUPS = [(12, 128, 6749, 1), (12, 128, 8001, 2), (12, 128, 13_001, 3), (12, 128, 20_001, 4),
+               (12, 128, 25_001, 6), (12, 128, 50_001, 12), (16, 128, 41_729, 4), (16, 64, 5087, 1),
+               (16, 64, 9001, 2), (16, 64, 20_001, 4), (16, 64, 39_805, 8), (16, 64, 60_001, 16), (12, 64, 20_001, 3)]
+
+
+@pytest.mark.parametrize("source", ["coords", "phases", "none"])
+@pytest.mark.parametrize("h,d,rows,hpb", HEAD_GROUPS)
+def test_k_transposed_every_head_group(dev, h, d, rows, hpb, source):
+    """Every head count per block and both head sizes, the first rows fetched
+    between positions and phases (coords) or after them (a phase table, no
+    RoPE), a ragged last tile and a tile of pads: equal to the row-major layout
+    (another kernel)."""
+    dtype = torch.bfloat16 if rows % 4 == 1 and hpb % 2 == 0 else torch.float16
+    g = torch.Generator(device=dev).manual_seed(rows + hpb)
+    k = torch.randn((rows, h, d), generator=g, device=dev).to(dtype)
+    coords = torch.randint(0, 64, (rows, 4), generator=g, device=dev, dtype=torch.int32)
+    gk = torch.randn((h, d), generator=g, device=dev) * 0.05 + 1
+    bk = torch.randn((h, d), generator=g, device=dev) * 0.02
+    fr = nn.rope_freqs(d)
+    kw = dict(bias_k=bk, gamma_q=gk, gamma_k=gk, lp=pad64(rows) + 64)
+    if source == "none":
+        kw.update(use_rope=False)
+    elif source == "phases":
+        kw.update(freqs=fr, phases=ops.rope_phases(rows, d, fr, coords=coords))
+    else:
+        kw.update(freqs=fr, coords=coords)
+    _, kt, _ = ops.attn_pack(None, k, None, k_transposed=True, **kw)
+    _, kn, _ = ops.attn_pack(None, k, None, k_transposed=False, **kw)
+    assert torch.equal(kt, kn.transpose(1, 2))
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])

@@ -34,6 +34,8 @@
 #include "t2h_internal.h"
 #include "t2h_rope.h"
 
+#include <cmath>
+
 namespace t2h {
 namespace {
 
@@ -175,10 +177,13 @@ __device__ __forceinline__ void transpose_to_tile(uint32_t (&w)[kPackIters][E / 
 // are requested between the positions' loads and the phases (39,804 x 12 x
 // 128: 60.9 -> 58.0 us), in 128 registers for 4 waves per SIMD. Blocks of one
 // head, in launches that are resident at once anyway, fetch after the phases
-// and keep their registers (2,369 rows: 9.8 against 10.4 us). Rows ahead of
-// the positions make the phases wait for them (62.8 us).
+// (2,369 rows: 9.8 against 10.4 us); with heads of 128 they are compiled for
+// one head, 89 registers instead of 146 and half the LDS, so that 5 fit a CU
+// and not 3 (4,246 rows, one head a block: 17.2 -> 13.6 us). Rows ahead of the
+// positions make the phases wait for them (62.8 us).
 template <typename T, int D, bool KT, bool AHEAD>
-__global__ __launch_bounds__(kPackBlock, AHEAD ? 4 : 1) void pack_tile_kernel(PackArgs a, RopeSlots tab, PackOrder order) {
+__global__ __launch_bounds__(kPackBlock, KT && sizeof(T) == 2 && (AHEAD || D == 128) ? 4 : 1)
+    void pack_tile_kernel(PackArgs a, RopeSlots tab, PackOrder order) {
     using L = HeadLanes<T, D>;
     constexpr int E = L::E;
     constexpr int P = L::P;
@@ -186,8 +191,10 @@ __global__ __launch_bounds__(kPackBlock, AHEAD ? 4 : 1) void pack_tile_kernel(Pa
     // 16-bit storage the output bit patterns in two buffers, so a head's tile
     // is written while the previous head's is read (one barrier per head).
     constexpr bool kTwo = KT && sizeof(T) == 2;
+    constexpr bool kOne = kTwo && !AHEAD && D == 128;
     __shared__ float tile[KT && !kTwo ? kPackRows : 1][KT && !kTwo ? D + 1 : 1];
-    __shared__ __attribute__((aligned(16))) uint8_t tile2[kTwo ? 2 : 1][kTwo ? D * kTileRow : 16];
+    __shared__ __attribute__((aligned(16))) uint8_t tile2[kTwo && !kOne ? 2 : 1][kTwo ? D * kTileRow : 16];
+    const int hpb = kOne ? 1 : order.hpb;
     const int lane = lane_id();
     const int g = lane >> 4;
     const int m = lane & 15;
@@ -255,7 +262,7 @@ __global__ __launch_bounds__(kPackBlock, AHEAD ? 4 : 1) void pack_tile_kernel(Pa
                 float pos[kPackIters][T2H_MAX_POS_DIM];
 #pragma unroll
                 for (int it = 0; it < kPackIters; ++it) src.get(rl[it], pos[it]);
-                fetch(hg * order.hpb);
+                fetch(hg * hpb);
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
                 for (int it = 0; it < kPackIters; ++it)
@@ -273,11 +280,11 @@ __global__ __launch_bounds__(kPackBlock, AHEAD ? 4 : 1) void pack_tile_kernel(Pa
         }
     }
     if constexpr (KT) {
-        if (!AHEAD || !rope || a.phases != nullptr) fetch(hg * order.hpb);
+        if (!AHEAD || !rope || a.phases != nullptr) fetch(hg * hpb);
     }
 
-    for (int zi = 0; zi < order.hpb; ++zi) {
-        const int z = hg * order.hpb + zi;
+    for (int zi = 0; zi < hpb; ++zi) {
+        const int z = hg * hpb + zi;
         if constexpr (!KT) fetch(z);
         float v[kPackIters][E];
         if (a.rows > 0) {
@@ -333,13 +340,13 @@ __global__ __launch_bounds__(kPackBlock, AHEAD ? 4 : 1) void pack_tile_kernel(Pa
             }
         }
         if constexpr (kTwo) {
-            uint8_t* buf = tile2[zi & 1];
+            uint8_t* buf = tile2[kOne ? 0 : zi & 1];
             transpose_to_tile<E>(pw, buf, wave, g, m);
             // this head's tile is whole, and every read of the tile written
             // two heads ago (the other buffer's previous contents) is done.
             // Only LDS is shared: the previous head's stores stay in flight
             lds_barrier();
-            if (zi + 1 < order.hpb) fetch(z + 1);
+            if (zi + 1 < hpb) fetch(z + 1);
             constexpr int VE = kPack<T>;
             constexpr int VPR = kPackRows / VE;
 #pragma unroll AHEAD ? 1 : D * VPR / kPackBlock
@@ -353,7 +360,7 @@ __global__ __launch_bounds__(kPackBlock, AHEAD ? 4 : 1) void pack_tile_kernel(Pa
             }
         } else if constexpr (KT) {
             __syncthreads();
-            if (zi + 1 < order.hpb) fetch(z + 1);
+            if (zi + 1 < hpb) fetch(z + 1);
             constexpr int VE = kPack<T>;            // elements per 16-byte vector
             constexpr int VPR = kPackRows / VE;     // vectors per output row (one e)
             for (int vi = threadIdx.x; vi < D * VPR; vi += kPackBlock) {
@@ -662,23 +669,28 @@ int heads_per_block(int64_t tiles, int tensors, int heads) {
     return best;
 }
 
-// The same for the 16-bit transposed k: the least modelled time, rounds of
-// resident blocks (4 per CU, 6 for head_dim 64, one less without AHEAD: registers) times a block's
-// fixed part (16 or 8 sincosf per lane, first loads) and its heads. us by
-// heads per block, 12 heads of 128: 9,000 rows 22.8 (1), 19.4 (2), 20.8 (4),
-// 24.2 (6), 35.7 (12); 39,804 rows 80.7, 63.4 (2), 61.5 (3), 58.2 (4), 64.7
-// (6), 56.6 (12); 120,000 rows 228, 172 (2), 158 (4), 155 (6), 154 (12). 16
-// heads of 64: 39,804 rows 41.9 (4), 38.3 (8), 44.9 (16); 100,000 rows 107
-// (4), 94.6 (8), 104 (16).
+// The same for the 16-bit transposed k: the least modelled time. A block
+// costs a fixed part (positions, phases, first loads: as much as 1.5 heads of
+// 128 or 3 of 64) and its heads; launches past one round of resident blocks
+// count their rounds between whole ones (0.4) and exact ones (0.6: blocks
+// drift apart), and half a block for the tail. Blocks of more than 1,536
+// channels are slower (16 heads of 128, 41,728 rows: 88 us, of 4 heads 80).
+// us by heads per block, 12 heads of 128: 4,100 rows 13.6 (1), 14.5 (2), 17.6
+// (4), 35.4 (12); 8,997 24.0, 20.0, 21.5, 36.3; 40,679 82.4, 64.8, 58.9, 57.0;
+// 75,000 rows 111 (2), 105 (4), 106 (6), 115 (12); 201,436 264 (3), 257 (4),
+// 257 (6), 275 (12). 16 heads of 64: 40,000 rows 42.1 (4), 38.5 (8), 46.5 (16);
+// 95,000 90.0, 86.7, 82.6. Over 270 sizes of 600 to 230,000 rows and 8 to 16
+// heads the choice is 0.2 % slower than the best on average, 6 % at most.
 int heads_per_block_kt(int64_t tiles, int heads, int head_dim) {
     int best = 1;
-    int64_t least = 0;
+    float least = 0.0f;
     for (int hpb = 1; hpb <= heads; ++hpb) {
-        if (heads % hpb) continue;
-        const int64_t resident = ((head_dim == 64 ? 6LL : 4LL) - (hpb == 1)) * device_cu_count();
-        const int64_t rounds = (tiles * (heads / hpb) + resident - 1) / resident;
-        const int64_t cost = rounds * (3 + hpb);
-        if (least == 0 || cost < least) {
+        if (heads % hpb || (hpb > 1 && hpb * head_dim > 1536)) continue;
+        const int per_cu = hpb == 1 ? 5 : head_dim == 64 ? 6 : 4;      // registers
+        const float rounds = (float)(tiles * (heads / hpb)) / (float)(per_cu * device_cu_count());
+        const float block = (head_dim == 64 ? 3.0f : 1.5f) + (float)hpb;
+        const float cost = block * (rounds <= 1.0f ? 1.0f : 0.6f * rounds + 0.4f * std::ceil(rounds) + 0.5f);
+        if (least == 0.0f || cost < least) {
             least = cost;
             best = hpb;
         }
