@@ -3,7 +3,9 @@
 // status. A call of 14 to 29 arguments through ctypes spends 3-4 us converting
 // them, as long as the launch itself; the calls of small token counts are
 // bound by that. bind(path) resolves the functions in the library the ctypes
-// binding has loaded. Conversions follow ctypes: integers wrap to their width.
+// binding has loaded. Integers wrap to their width as in ctypes; what is refused
+// here with a TypeError or OverflowError (ctypes objects, say), before the
+// function is called, the caller passes to the ctypes binding.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 #include <dlfcn.h>
@@ -20,6 +22,10 @@ namespace {
 template <typename T> T arg(PyObject* o) {
     if constexpr (std::is_pointer<T>::value) {
         if (o == Py_None) return nullptr;
+        if (!PyLong_Check(o)) {
+            PyErr_Format(PyExc_TypeError, "pointer must be an int or None, not %.100s", Py_TYPE(o)->tp_name);
+            return nullptr;
+        }
         return reinterpret_cast<T>(static_cast<uintptr_t>(PyLong_AsUnsignedLongLongMask(o)));
     } else if constexpr (std::is_floating_point<T>::value) {
         return static_cast<T>(PyFloat_AsDouble(o));

@@ -125,6 +125,9 @@ def call(name: str, *args) -> None:
     if f is None:
         load()
         f = _calls[name]
-    rc = f(*args)
+    try:
+        rc = f(*args)
+    except (TypeError, OverflowError):      # ctypes takes more argument forms, and refuses the others its own way
+        rc = getattr(_lib, name)(*args)
     if rc != T2H_OK:
         check(rc)
