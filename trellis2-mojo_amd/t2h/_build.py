@@ -2,15 +2,17 @@
 
 Each csrc/*.hip translation unit is compiled in parallel, then linked into
 lib/libt2h.so next to this package; csrc/t2h_pycall.cpp (host code only)
-becomes lib/_t2h_pycall.so, the Python call module. The packed-FP32 target feature is turned
-off for every HIP compile (the host pass warns that it does not know the
-feature; that warning is filtered).
+becomes the Python call module of this interpreter, if it has its headers and
+there is a C++ compiler (without it calls go through ctypes). The packed-FP32
+target feature is turned off for every HIP compile (the host pass warns that it
+does not know the feature; that warning is filtered).
 """
 from __future__ import annotations
 
 import concurrent.futures as cf
 import glob
 import os
+import shutil
 import subprocess
 import sysconfig
 
@@ -21,7 +23,8 @@ INCLUDE = os.path.join(REPO_ROOT, "include")
 BUILD_DIR = os.path.join(PKG_ROOT, "_build")
 LIB_DIR = os.path.join(PKG_ROOT, "lib")
 LIB_PATH = os.path.join(LIB_DIR, "libt2h.so")
-PYCALL_PATH = os.path.join(LIB_DIR, "_t2h_pycall.so")
+# the interpreter's tag is in the name: another Python does not load it
+PYCALL_PATH = os.path.join(LIB_DIR, "_t2h_pycall" + sysconfig.get_config_var("EXT_SUFFIX"))
 
 CXX = os.environ.get("CXX", "g++")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -58,10 +61,14 @@ def build(verbose: bool = False) -> str:
     # emitted) fails the link here instead of the first dlopen on a GPU box
     logs.append(_run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-Wl,-z,defs", *objs, "-o", tmp]))
     os.replace(tmp, LIB_PATH)
-    tmp = PYCALL_PATH + ".tmp"
-    logs.append(_run([CXX, "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", f"-I{INCLUDE}",
-                      f"-I{sysconfig.get_paths()['include']}", os.path.join(CSRC, "t2h_pycall.cpp"), "-ldl", "-o", tmp]))
-    os.replace(tmp, PYCALL_PATH)
+    pyinc = sysconfig.get_paths()["include"]
+    if os.path.exists(os.path.join(pyinc, "Python.h")) and shutil.which(CXX):
+        tmp = PYCALL_PATH + ".tmp"
+        logs.append(_run([CXX, "-O2", "-std=c++17", "-fPIC", "-Wall", "-shared", f"-I{INCLUDE}", f"-I{pyinc}",
+                          os.path.join(CSRC, "t2h_pycall.cpp"), "-ldl", "-o", tmp]))
+        os.replace(tmp, PYCALL_PATH)
+    elif os.path.exists(PYCALL_PATH):       # of an earlier build: its functions may differ
+        os.remove(PYCALL_PATH)
     if verbose:
         print("\n".join(l for l in logs if l.strip()))
     return LIB_PATH

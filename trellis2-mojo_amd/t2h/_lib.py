@@ -2,9 +2,9 @@
 
 The library is loaded once, after torch (so torch's HIP runtime — SONAME
 libamdhip64.so.7 — is the one the library binds to and device pointers are
-shared). There is no fallback: if the library or the call module
-(_t2h_pycall.so, the same functions without ctypes' conversions) is missing
-every op raises.
+shared). There is no fallback: if the library is missing every op raises. The
+call module (_t2h_pycall, the same functions without ctypes' conversions) takes
+the calls where it is built for this interpreter.
 """
 from __future__ import annotations
 
@@ -87,7 +87,7 @@ def load(path: str | None = None):
     if _lib is not None:
         return _lib
     import torch  # noqa: F401  (bind to torch's HIP runtime first)
-    path = path or LIB_PATH
+    path = os.fsdecode(path or LIB_PATH)
     if not os.path.exists(path):
         raise RuntimeError(f"libt2h.so not found at {path}: run __graft_entry__.build() first")
     L = ctypes.CDLL(path)
@@ -101,13 +101,14 @@ def load(path: str | None = None):
         fn = getattr(L, name)
         fn.restype = c_i32
         fn.argtypes = args
-    if not os.path.exists(PYCALL_PATH):
-        raise RuntimeError(f"_t2h_pycall.so not found at {PYCALL_PATH}: run __graft_entry__.build() first")
-    loader = importlib.machinery.ExtensionFileLoader("_t2h_pycall", PYCALL_PATH)
-    m = importlib.util.module_from_spec(importlib.util.spec_from_loader("_t2h_pycall", loader))
-    loader.exec_module(m)
-    m.bind(path)
-    _calls.update((name, getattr(m, name, None) or getattr(L, name)) for name in _SIGNATURES)
+    calls = {name: getattr(L, name) for name in _SIGNATURES}
+    if os.path.exists(PYCALL_PATH):
+        loader = importlib.machinery.ExtensionFileLoader("_t2h_pycall", PYCALL_PATH)
+        m = importlib.util.module_from_spec(importlib.util.spec_from_loader("_t2h_pycall", loader))
+        loader.exec_module(m)
+        m.bind(path)
+        calls.update((name, getattr(m, name)) for name in _SIGNATURES if hasattr(m, name))
+    _calls.update(calls)
     _lib = L
     return L
 

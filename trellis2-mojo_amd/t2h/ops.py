@@ -23,10 +23,16 @@ ACT_NONE = -1
 OP_ADD, OP_SUB, OP_MUL, OP_DIV, OP_RSUB, OP_RDIV = 0, 1, 2, 3, 4, 5
 
 
+# not a documented function of torch
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) if hasattr(torch._C, "_cuda_getDevice") else None
+
+
 def _stream() -> int:
     """torch's current stream on the current device (the handle alone: the
     Stream object of torch.cuda.current_stream() takes 1.5 us to make)."""
-    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+    if _raw_stream is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(torch._C._cuda_getDevice())
 
 
 def _ptr(t: Optional[torch.Tensor]):
