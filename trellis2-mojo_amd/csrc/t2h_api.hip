@@ -413,7 +413,6 @@ int32_t t2h_attn_pack(const void* q, const void* k, const void* v, int64_t in_st
     a.q_scale = 1.0f / std::sqrt((float)head_dim);      // attention.mojo:587
     a.use_rope = use_rope ? 1 : 0;
     a.pos_dim = pos_dim;
-    a.freq_dim = use_rope ? freq_dim : 0;
     a.phases = use_rope ? phases : nullptr;
     a.phase_rows = phase_rows;
     a.coords = (use_rope && phases == nullptr) ? coords : nullptr;

@@ -96,7 +96,7 @@ struct PackArgs {
     float q_scale;           // 1 / f32 sqrt(head_dim), baked into qh
     int32_t use_rope;
     int32_t pos_dim;
-    int32_t freq_dim;        // distinct rotary frequencies
+    int32_t freq_dim;        // distinct rotary frequencies (t2h_qkv_linear_pack)
     const float* phases;
     int64_t phase_rows;
     const int32_t* coords;
