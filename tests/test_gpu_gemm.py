@@ -33,7 +33,7 @@ def _sum_bound(a, w):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_integer_operands_bit_exact(dev, dtype):
-    """Small-integer operands, ragged rows (300 = 2 token tiles + 44): every
+    """Small-integer operands, ragged rows (300 = 4 token tiles of 64 + 44): every
     output equals the oracle bit for bit; pins the MFMA operand and output
     lane layouts and the tile bookkeeping."""
     rng = np.random.default_rng(11)
@@ -43,7 +43,7 @@ def test_integer_operands_bit_exact(dev, dtype):
     out = ops.linear(to_dev(a, dev, dtype), to_dev(w, dev, dtype), out_dtype=torch.float32)
     want = orc.linear(a, w)
     assert np.array_equal(host(out), want)
-    # 16-bit output (the LDS-staged row store): |sums| < 256 are exact in f16
+    # 16-bit output: |sums| < 256 are exact in f16
     # and bf16 needs |sums| < 256 too, so clip the operands
     a2, w2 = np.clip(a, -2, 2), np.clip(w, -2, 2)
     out16 = ops.linear(to_dev(a2, dev, dtype), to_dev(w2, dev, dtype))
@@ -54,7 +54,7 @@ def test_integer_operands_bit_exact(dev, dtype):
 
 @pytest.mark.parametrize("out_dtype,act", [(torch.float32, None), (torch.float16, ops.ACT_RELU)])
 def test_more_tiles_than_cus_bit_exact(dev, out_dtype, act):
-    """66 token tiles (the last one ragged: 16740 = 65 * 256 + 100) x 7
+    """66 token tiles of 256 (the last one ragged: 16740 = 65 * 256 + 100) x 7
     feature tiles = 462 tiles: more than one per CU, and a count that is not
     a multiple of 8, so the XCD deal of the tile numbers has unequal ranges.
     Integer operands and bias, |sums| <= 772, so f32 and f16 outputs (ReLU
@@ -73,8 +73,8 @@ def test_more_tiles_than_cus_bit_exact(dev, out_dtype, act):
 
 def test_long_k_tile_order_bit_exact(dev):
     """K = 4096 (64 k steps; the tile order groups 2 token tiles instead of
-    4) with 3 token tiles, the last ragged: a group of 2 and a remainder of
-    1. Operands in {-1, 0, 1}: exact sums, |sums| < 2048, so both the f32
+    4) on 32 x 64 tiles, 10 token tiles, the last ragged (256 x 256 tiles:
+    test_gpu_gemm_tiles.py). Operands in {-1, 0, 1}: exact sums, |sums| < 2048, so both the f32
     and the f16 output equal the oracle bit for bit, as does the gated
     residual join on the same GEMM."""
     rng = np.random.default_rng(29)
@@ -217,9 +217,8 @@ def test_gate_residual_ungated_no_bias_f16(dev):
 
 @pytest.mark.parametrize("k", [64, 128, 192])
 def test_one_two_three_k_steps_bit_exact(dev, k):
-    """1, 2 and 3 k steps of 64 (the pipelines' prologue and tails, and the
-    stage buffer the last step leaves free for the residual rows, which
-    alternates with the step count): integer operands, bit-exact, for the
+    """1, 2 and 3 k steps of 64 (fewer than the 32 x 64 tiles' stages; every
+    tile size: test_gpu_gemm_tiles.py): integer operands, bit-exact, for the
     linear (f32 and 16-bit out) and the gated residual (f16 and f32 streams)."""
     m, n = 300, 512
     rng, a, w = _int_case(30 + k, m, n, k, -2, 3)

@@ -16,9 +16,10 @@ from t2h import nn, ops
 
 pytestmark = pytest.mark.gpu
 
-# one row count per tile size for N = 1536 on 256 CUs (32 x 64, 64 x 64,
-# 128 x 64, 128 x 128, 256 x 128, 256 x 256, the last with more tiles than CUs),
-# none a multiple of its tile
+# row counts, none a multiple of its tile, that at N = 1536 and K = 128 or 192
+# take 32 x 64 (two), 64 x 64, 128 x 64, 128 x 128, 256 x 128, 256 x 256 and
+# 256 x 128 tiles on 256 CUs, the last two or three to a block. (At K = 1536
+# the last takes 256 x 256.)
 ROWS = [1, 301, 501, 1001, 2001, 4101, 8001, 12001]
 
 
@@ -62,11 +63,56 @@ def test_gate_residual_every_tile_exact(dev, rows, res_dtype):
 @pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 1536])
 @pytest.mark.parametrize("rows", [9, 700, 2100, 9000])
 def test_k_steps_exact(dev, rows, k):
-    """One step to many, odd and even, on tiles of every stage depth."""
+    """One step to many, odd and even, on 32 x 64 (two row counts), 128 x 64
+    and 256 x 128 tiles (every size: test_every_tile_at_few_k_steps)."""
     rng = np.random.default_rng(k + rows)
     a, w = _signs(rng, (rows, k)), _signs(rng, (512, k))
     got = ops.linear(to_dev(a, dev, torch.float16), to_dev(w, dev, torch.float16), out_dtype=torch.float32)
     assert np.array_equal(host(got), orc.linear(a, w))
+
+
+def _exact(a, w, b=None):
+    """a w^T + b of small integers: exact in f32 in any order."""
+    out = a @ w.T
+    return out if b is None else out + b
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 320, 448])
+@pytest.mark.parametrize("rows", [9, 1501, 3001, 6001, 12_001, 16_501])
+def test_every_tile_at_few_k_steps(dev, rows, k):
+    """N = 512: 32 x 64, 64 x 64, 128 x 64, 128 x 128, 256 x 128 and 256 x 256
+    tiles at 1 to 7 k steps: fewer than their stages, odd and even, the linear
+    and the residual in both stream types."""
+    rng = np.random.default_rng(1000 + k + rows)
+    a, w, b = _signs(rng, (rows, k)), _signs(rng, (512, k)), rng.integers(-3, 4, (512,)).astype(np.float32)
+    ad, wd, bd = to_dev(a, dev, torch.float16), to_dev(w, dev, torch.float16), to_dev(b, dev)
+    want = _exact(a, w, b)
+    assert np.array_equal(host(ops.linear(ad, wd, bd, out_dtype=torch.float32)), want)
+    assert np.array_equal(host(ops.linear(ad, wd, bd)), want)
+    res = rng.integers(-8, 9, (rows, 512)).astype(np.float32)
+    for dt in (torch.float16, torch.float32):
+        assert np.array_equal(host(ops.linear_gate_residual(ad, wd, to_dev(res, dev, dt), bias=bd)), res + want)
+
+
+@pytest.mark.parametrize("res_dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,k", [(16_741, 192), (12_001, 192), (16_741, 4096)])
+def test_residual_of_several_tiles_per_block(dev, rows, k, res_dtype):
+    """396 tiles of 256 x 256 (564 of 256 x 128 at 12,001 rows) on 256 CUs: a
+    block's residual rows, gate row and next operands overlap from tile to
+    tile. Batches end inside tiles and at their edges, the join is in place;
+    K = 4096 groups two token tiles instead of four."""
+    rng = np.random.default_rng(2000 + rows + k)
+    n = 1536
+    a, w, b = _signs(rng, (rows, k)), _signs(rng, (n, k)), rng.integers(-3, 4, (n,)).astype(np.float32)
+    cuts = np.array([0, 100, 256, 5000, 5000, 2 * rows // 3, rows], np.int64)
+    gate = (2.0 ** rng.integers(-1, 2, (6, n))).astype(np.float32)
+    res = rng.integers(-8, 9, (rows, n)).astype(np.float32)
+    want = res + _exact(a, w, b) * np.repeat(gate, np.diff(cuts), axis=0)
+    assert np.abs(want).max() < 1024                       # halves are exact in f16
+    rd = to_dev(res, dev, res_dtype)
+    ops.linear_gate_residual(to_dev(a, dev, torch.float16), to_dev(w, dev, torch.float16), rd, bias=to_dev(b, dev),
+                             gate=to_dev(gate, dev), offsets=to_dev(cuts, dev), out=rd)
+    assert np.array_equal(host(rd), want)
 
 
 def test_rows_do_not_depend_on_the_row_count(dev):
@@ -92,6 +138,11 @@ def test_row_strides_past_32_bit_offsets(dev):
     for got, want in zip(ops.qkv_linear_pack(x, w, 2, use_rope=False, mp=8, lp=8),
                          ops.qkv_linear_pack(x.contiguous(), w, 2, use_rope=False, mp=8, lp=8)):
         assert torch.equal(got, want)
+    gate = torch.randn((1, 768), generator=g, device=dev)
+    for dt in (torch.float16, torch.float32):
+        res = torch.randn((rows, 768), generator=g, device=dev).to(dt)
+        assert torch.equal(ops.linear_gate_residual(x, w, res, gate=gate),
+                           ops.linear_gate_residual(x.contiguous(), w, res, gate=gate))
 
 
 @pytest.mark.parametrize("rows", [70, 1700, 3001])
@@ -99,8 +150,9 @@ def test_row_strides_past_32_bit_offsets(dev):
 @pytest.mark.parametrize("kt", [True, False])
 def test_qkv_positions_in_and_out_of_the_lookup(dev, rows, heads, hd, kt):
     """cos/sin looked up in the block's table, and computed for tokens whose
-    coordinates it does not hold (negative, 128, large): the same bits as from
-    the phase table of the same coordinates."""
+    coordinates it does not hold (negative, 5,000): the same bits as from the
+    phase table of the same coordinates. 128-token tiles, one to a block (the
+    others: test_gpu_qkv_positions.py)."""
     rng = np.random.default_rng(rows + hd)
     c = rng.integers(0, 128, (rows, 4)).astype(np.int32)
     odd = rng.choice(rows, rows // 9, replace=False)

@@ -46,7 +46,7 @@ def close_where_finite(got, want, tol, what):
     return int(fin.size - fin.sum())
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_layernorm_modulate_nonfinite_rows(dev, dtype):
     rows, c = 16, 1536
     x = orc.randn(901, (rows, c))
@@ -96,7 +96,7 @@ def test_qk_rmsnorm_rope_nonfinite_heads(dev):
     assert np.all(np.isfinite(wq[[0, 4, 5, 6, 7]])) and np.all(np.isfinite(wk[[0, 1, 2, 3, 6, 7]]))
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_gelu_tanh_bias_nonfinite(dev, dtype):
     specials = [np.nan, np.inf, -np.inf, 0.0, -0.0, 20.0, -20.0, 88.0, -88.0]
     if dtype == torch.float32:
@@ -118,7 +118,7 @@ def test_gelu_tanh_bias_nonfinite(dev, dtype):
     assert np.isposinf(got[0, 1]) and np.isnan(got[0, 2])
 
 
-@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
 def test_gated_residual_nonfinite(dev, dtype):
     rows, c = 8, 1536
     x = orc.randn(931, (rows, c))
