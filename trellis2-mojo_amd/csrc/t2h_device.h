@@ -29,7 +29,7 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint32_t b16) {
 
 // f32 -> bf16 bits, round to nearest even, NaN kept quiet: v_cvt_pk_bf16_f32,
 // one instruction per pair where the same in integer arithmetic took seven
-// per value (checked equal over all 2^32 inputs).
+// per value (the same bits: tests/test_gpu_bf16_rounding.py).
 __device__ __forceinline__ uint32_t f32_to_bf16_bits(float f) {
     return (uint32_t)__builtin_bit_cast(uint16_t, (__bf16)f);
 }
@@ -162,10 +162,16 @@ template <> __device__ __forceinline__ float ld1<__bf16>(const __bf16* p) {
 // gated-residual thread's eight) uses the default cache policy instead:
 // LN + modulate 201 -> 188 us, the config-5 chain 1,628 -> 1,601 us. All
 // non-temporal, or all cached, is slower. Launches that move less than
-// T2H_CACHED_SHARE_MIN bytes keep every load non-temporal. The line from 512
-// to 100 MB: a block's glue (LN, two joins, residual) over 39,804 f16 rows 277
-// -> 265 us, 20,000 150.5 -> 146, 9,000 f32 rows 140 -> 137; launches below
-// 100 MB were the same with and without.
+// T2H_CACHED_SHARE_MIN bytes keep every load non-temporal: below 100 MB the
+// share made no difference. From there on it is a gain or equal behind kernels
+// that store non-temporally, as this library's do (f16, 39,804 rows: the join +
+// LN after the out projection 88.7 -> 84.4 us, LN after the qkv pack 47.0 ->
+// 44.3; a block's glue 277 -> 265), and equal behind torch's projections and
+// MLP. It is a loss behind a kernel that has just filled the infinity cache with
+// ordinary stores to other memory, which the share's lines then push out: LN of
+// 110 MB and a 320 MB fill before it 74.0 -> 80.8 us together, of 500 MB 138 ->
+// 154; with a 200 MB fill 0-5 %, with 100 MB or less none. That holds on either
+// side of the line.
 #ifndef T2H_CACHED_SHARE_MIN
 #define T2H_CACHED_SHARE_MIN (int64_t(100) << 20)
 #endif

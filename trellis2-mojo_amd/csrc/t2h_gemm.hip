@@ -363,10 +363,12 @@ hipError_t qkv_typed(GemmArgs g, const PackArgs& p, const RopeSlots& tab, int64_
     return hipGetLastError();
 }
 
-// 128-token tiles when 256-token ones would occupy half of the CUs at most
-// (each then takes 0.7 of the time: 1,200 tokens x 4608 features on 180 tiles
-// and not 90); 256 otherwise (2,369 tokens: 180 tiles of 256, 33 us; 342 of
-// 128, 45 us).
+// 128-token tiles when 256-token ones would occupy half of the CUs at most;
+// 256 otherwise. us back to back, f16, 4608 features of K = 1536, with bias,
+// RMS and RoPE from coordinates (without RMS and RoPE): 1,200 tokens 33.5 (26.4)
+// on 180 tiles of 128, 45.8 (33.7) on 90 of 256; 2,369 tokens 47.6 (36.0) on
+// 180 of 256, 60.4 (48.9) on 342 of 128. From 3,600 to 5,000 tokens 128 would be
+// 3-8 % faster with RMS and RoPE, 2-3 % slower without.
 template <typename T, int HD>
 hipError_t qkv_sized(const GemmArgs& g, const PackArgs& p, const RopeSlots& tab, int64_t span, hipStream_t s) {
     if (g.ldx > kMaxStride32 || g.k > kMaxStride32) return qkv_typed<T, HD, 128, true>(g, p, tab, span, s);

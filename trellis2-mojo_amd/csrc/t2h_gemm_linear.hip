@@ -258,16 +258,18 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_res_kernel(GemmArgs a) {
 // stages of 32 * KK k are filled by direct-to-LDS loads up to NST - 1 stages
 // ahead; a step's fragments are read while the previous step's MFMAs run, and
 // one barrier per step both publishes a stage and frees one. What bounds it is
-// the LDS (a small tile reuses little) and the latency of a step. 2,369 tokens
-// (f16), 256 x 256 tiles against these: K = 6144 to 1536 features 92 -> 50 us
-// (228 tiles of 128 x 128 instead of 60), K = 1536 to 1536 27.7 -> 16; 1,029
-// tokens, K = 1024 to 3072: 20 -> 12; 16 tokens, K = 1536 to 9216: 26.6 -> 7.2.
+// the LDS (a small tile reuses little) and the latency of a step. us a launch,
+// back to back on one set of operands (f16, bias), 256 x 256 tiles against
+// these: 2,369 tokens, K = 6144 to 1536 features 95 -> 50 (228 tiles of 128 x
+// 128 instead of 60; 62 as one launch of an MLP), K = 1536 to 1536 29.5 -> 17.7;
+// 1,029 tokens, K = 1024 to 3072 22 -> 13.7; one token, K = 1536 to 9216, on 64
+// x 64 7.6, on 256 x 128 21.
 // The sums run over k in the main loop's order on every tile size, so a row's
 // result depends neither on the row count nor on the kernel. (Splitting k over
 // two or four groups of waves and adding through LDS was no faster.)
 // W64: 64-bit operand offsets (row strides past kMaxStride32).
 template <int BF, int BT, int WF, int WT, int KK, int NST> struct Small {
-    static constexpr int kWaves = WF * WT, kThr = 64 * kWaves;
+    static constexpr int kWaves = WF * WT;
     static constexpr int kSK = 32 * KK;                 // k per stage
     static constexpr int kNB = kSK / kBK;               // 64-k blocks per stage
     static constexpr int kFI = BF / WF / 16, kTJ = BT / WT / 16;
@@ -437,10 +439,15 @@ hipError_t launch_small(GemmArgs a, hipStream_t s) {
 // Tile choice: the least modelled time, rounds * (base + perk * K / 1024) us
 // for rounds = ceil(tiles / CUs). The constants are least-squares readings of
 // each tile timed over 1 to 20,000 rows, K 256 to 6,144 and N 1,024 to 9,216
-// (f16; within 10 % of the measured times of launches of one to three rounds):
-// small tiles win while the larger ones leave CUs idle, large ones where all
-// are busy, e.g. N = K = 1536: 32 x 64 to ~340 rows, 64 x 64 to ~680, 128 x 64
-// to ~1,360, 128 x 128 to ~2,700, 256 x 128 to ~5,400, then 256 x 256.
+// (f16, no epilogue): small tiles win while the larger ones leave CUs idle,
+// large ones where all are busy, e.g. N = K = 1536: 32 x 64 to ~340 rows, 64 x
+// 64 to ~680, 128 x 64 to ~1,360, 128 x 128 to ~2,700, 256 x 128 to ~5,400,
+// then 256 x 256. It ranks the tiles and is no prediction: launches of one to
+// three rounds, 1 to 39,804 rows at seven (N, K), measured 4 % below to 49 %
+// above it (bias, GELU, f32 output; mean 22 %), to 70 % with a 16-bit residual
+// and 137 % with an f32 one. The choice was the fastest tile within 0.3 %
+// without a residual, within 8 % (0.2 % on average) with a 16-bit residual and
+// within 21 % (1.5 %) with an f32 one, whose epilogue costs the large tiles more.
 enum GemmPlan { kPlanBig, kPlan128, kPlan128x64, kPlan64, kPlan32x64, kPlanBig128, kPlanWide };
 struct PlanCost {
     GemmPlan plan;
