@@ -872,13 +872,15 @@ TRAFFIC_COMMON = ["t2h_device.h", "t2h_internal.h"]
 
 
 def traffic_sources_sha(op):
-    """sha256 over the csrc files `op`'s kernel is built from, in a fixed order."""
+    """sha256 over the code of the csrc files `op`'s kernel is built from, in a
+    fixed order (comments and blank lines do not change a kernel's traffic)."""
     import hashlib
 
     h = hashlib.sha256()
     for f in TRAFFIC_SOURCES[op] + TRAFFIC_COMMON:
-        with open(os.path.join(ROOT, "trellis2-mojo_amd", "csrc", f), "rb") as fh:
-            h.update(f.encode() + b"\0" + fh.read())
+        with open(os.path.join(ROOT, "trellis2-mojo_amd", "csrc", f), encoding="utf-8") as fh:
+            code = [line.split("//")[0].rstrip() for line in fh]
+        h.update((f + "\0" + "\n".join(c for c in code if c)).encode())
     return h.hexdigest()
 
 

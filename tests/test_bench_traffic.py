@@ -36,6 +36,14 @@ def test_missing_file_or_op(tmp_path):
     assert bench.measured_traffic("ln_modulate", p) == (None, False)
 
 
+def test_committed_figures_belong_to_the_sources():
+    """A change to a chain kernel's code needs its counters read again
+    (profiles/chain_c5_traffic_pmc.md has the commands)."""
+    for op in bench.TRAFFIC_SOURCES:
+        figure, stale = bench.measured_traffic(op)
+        assert not stale and figure > 0, op
+
+
 def test_fingerprint_covers_each_source():
     # every op's fingerprint names existing files, and ops on different
     # kernels get different fingerprints
