@@ -101,7 +101,7 @@ def test_k_layouts_agree(dev, dtype, d):
 def test_k_transposed_head_groups(dev, dtype, rows):
     """The transposed-k tile kernel walks a group of heads per block, the
     16-bit tiles alternating between two LDS buffers from head to head. On
-    256 CUs these row counts give 6, 4, 4 and 6 heads per block (the others:
+    256 CUs these row counts give 6, 12, 4 and 6 heads per block (the others:
     test_k_transposed_every_head_group); each must equal the row-major layout
     (another kernel) exactly."""
     h, d = 12, 128

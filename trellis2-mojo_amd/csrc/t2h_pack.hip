@@ -175,12 +175,12 @@ __device__ __forceinline__ void transpose_to_tile(uint32_t (&w)[kPackIters][E / 
 
 // AHEAD (16-bit transposed k, blocks of several heads): the first head's rows
 // are requested between the positions' loads and the phases (39,804 x 12 x
-// 128: 60.9 -> 58.0 us), in 128 registers for 4 waves per SIMD. Blocks of one
-// head, in launches that are resident at once anyway, fetch after the phases
-// (2,369 rows: 9.8 against 10.4 us); with heads of 128 they are compiled for
-// one head, 89 registers instead of 146 and half the LDS, so that 5 fit a CU
-// and not 3 (4,246 rows, one head a block: 17.2 -> 13.6 us). Rows ahead of the
-// positions make the phases wait for them (62.8 us).
+// 128, 4 heads a block: 60.9 -> 58.0 us), in 128 registers for 4 waves per
+// SIMD. Blocks of one head, in launches that are resident at once anyway, fetch
+// after the phases (2,369 rows: 9.8 against 10.4 us); with heads of 128 they
+// are compiled for one head, 89 registers instead of 146 and half the LDS, so
+// that 5 fit a CU and not 3 (4,246 rows, one head a block: 17.2 -> 13.6 us).
+// Rows ahead of the positions make the phases wait for them (62.8 us).
 template <typename T, int D, bool KT, bool AHEAD>
 __global__ __launch_bounds__(kPackBlock, KT && sizeof(T) == 2 && (AHEAD || D == 128) ? 4 : 1)
     void pack_tile_kernel(PackArgs a, RopeSlots tab, PackOrder order) {
@@ -672,8 +672,8 @@ int heads_per_block(int64_t tiles, int tensors, int heads) {
 // The same for the 16-bit transposed k: the least modelled time. A block
 // costs a fixed part (positions, phases, first loads: as much as 1.5 heads of
 // 128 or 3 of 64) and its heads; launches past one round of resident blocks
-// count their rounds between whole ones (0.4) and exact ones (0.6: blocks
-// drift apart), and half a block for the tail. Blocks of more than 1,536
+// count their rounds between exact ones (0.4: blocks drift apart) and whole
+// ones (0.6), and 0.6 of a block for the tail. Blocks of more than 1,536
 // channels are slower (16 heads of 128, 41,728 rows: 88 us, of 4 heads 80).
 // us by heads per block, 12 heads of 128: 4,100 rows 13.6 (1), 14.5 (2), 17.6
 // (4), 35.4 (12); 8,997 24.0, 20.0, 21.5, 36.3; 40,679 82.4, 64.8, 58.9, 57.0;
@@ -689,7 +689,7 @@ int heads_per_block_kt(int64_t tiles, int heads, int head_dim) {
         const int per_cu = hpb == 1 ? 5 : head_dim == 64 ? 6 : 4;      // registers
         const float rounds = (float)(tiles * (heads / hpb)) / (float)(per_cu * device_cu_count());
         const float block = (head_dim == 64 ? 3.0f : 1.5f) + (float)hpb;
-        const float cost = block * (rounds <= 1.0f ? 1.0f : 0.6f * rounds + 0.4f * std::ceil(rounds) + 0.5f);
+        const float cost = block * (rounds <= 1.0f ? 1.0f : 0.4f * rounds + 0.6f * std::ceil(rounds) + 0.6f);
         if (least == 0.0f || cost < least) {
             least = cost;
             best = hpb;
