@@ -1,4 +1,4 @@
-"""Launches past 100 MB read a small share of their rows with the default
+"""Launches past 512 MB read a small share of their rows with the default
 cache policy instead of the non-temporal one (LN + modulate and the fused
 join + LN: each row's first 1 KB piece; the gated residual: each tile's
 first residual row). The policy changes only how the bytes travel, so a
@@ -14,7 +14,7 @@ from t2h import ops
 pytestmark = pytest.mark.gpu
 
 C = 1536
-LIMIT = 100 << 20   # the library's threshold, in bytes moved per launch
+LIMIT = 512 << 20   # the library's threshold, in bytes moved per launch
 
 
 def _rows_over(nbytes_per_row):

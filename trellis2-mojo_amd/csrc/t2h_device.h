@@ -162,18 +162,17 @@ template <> __device__ __forceinline__ float ld1<__bf16>(const __bf16* p) {
 // gated-residual thread's eight) uses the default cache policy instead:
 // LN + modulate 201 -> 188 us, the config-5 chain 1,628 -> 1,601 us. All
 // non-temporal, or all cached, is slower. Launches that move less than
-// T2H_CACHED_SHARE_MIN bytes keep every load non-temporal: below 100 MB the
-// share made no difference. From there on it is a gain or equal behind kernels
+// T2H_CACHED_SHARE_MIN bytes keep every load non-temporal: the share's lines
+// push dirty lines of earlier kernels out of the 256 MB infinity cache, and the
+// launch waits for those writes. With the line at 100 MB, behind a fill that
+// left the cache dirty, LN over 39,804 f32 rows took 99.5-100.4 us instead of
+// 88.5 and the gated residual over 32,768 f16 rows 56.1 instead of 50.5 (warm:
+// 84 instead of 86.4, 47.1 instead of 48.3). It is a gain only behind kernels
 // that store non-temporally, as this library's do (f16, 39,804 rows: the join +
-// LN after the out projection 88.7 -> 84.4 us, LN after the qkv pack 47.0 ->
-// 44.3; a block's glue 277 -> 265), and equal behind torch's projections and
-// MLP. It is a loss behind a kernel that has just filled the infinity cache with
-// ordinary stores to other memory, which the share's lines then push out: LN of
-// 110 MB and a 320 MB fill before it 74.0 -> 80.8 us together, of 500 MB 138 ->
-// 154; with a 200 MB fill 0-5 %, with 100 MB or less none. That holds on either
-// side of the line.
+// LN after the out projection 88.7 -> 84.4, a block's glue 277 -> 265), and
+// neither behind torch's projections.
 #ifndef T2H_CACHED_SHARE_MIN
-#define T2H_CACHED_SHARE_MIN (int64_t(100) << 20)
+#define T2H_CACHED_SHARE_MIN (int64_t(512) << 20)
 #endif
 
 // E elements of T (E * sizeof(T) == 16) at element `off` of a wave-uniform
