@@ -17,8 +17,8 @@
 // GpuLinear.try_build 430-465); only the summation order differs.
 //
 // The main loop here (256 features x BT tokens, 8 waves) serves the large
-// launches: MI355X runs them at its power limit (1.5-1.8 GHz instead of 2.4),
-// so what counts is matrix-core work per joule and no idle matrix cores.
+// launches: MI355X runs them at its power limit (1.46-1.73 GHz over the four
+// large products of a 201,436-token block instead of 2.4), so what counts is matrix-core work per joule and no idle matrix cores.
 // - 16x16x32 MFMAs: a 256 x 256 tile of K = 6144 ran at 1,388 TFLOP/s with
 //   them and at 1,160 with 32x32x16 in the same loop (f16, 201,436 tokens).
 // - Direct-to-LDS loads (16 bytes per lane), no register staging.
@@ -26,13 +26,15 @@
 //   MFMAs (one 64-feature half of its wave tiles over 64 k) the other reads
 //   its next fragments and issues the loads of two steps ahead; a barrier ends
 //   each turn. 32 MFMAs a turn and not 16: 1,385 against 1,290 TFLOP/s. The
-//   matrix cores are busy 83 % of the loop; the plain two-waves-per-SIMD
-//   schedule that this replaced had 60-69 %.
+//   matrix cores are busy 70-72 % of a plain linear of K = 1536 (the two waves
+//   per SIMD in step that this replaced: 66-67 %) and 76-78 % of K = 6144 with
+//   the residual, epilogues included.
 // - Persistent blocks: the next tile's first loads are issued before this
 //   tile's epilogue (K = 1536: 1,284 -> 1,315 TFLOP/s).
-// In all, at 201,436 tokens (f16): K = 1536 to 6144 features 1,075 -> 1,250
-// TFLOP/s, K = 6144 to 1536 features 1,190 -> 1,315-1,360 (hipBLASLt on the
-// same boxes 1,270 and 1,330).
+// In all, at 201,436 tokens (f16, the former kernels and these in turn): K =
+// 1536 to 6144 features 1,115 -> 1,253 TFLOP/s (hipBLASLt 1,257), with bias and
+// GELU-tanh 1,022 -> 1,157-1,179; K = 6144 to 1536 features 1,212 -> 1,355
+// (1,343), with the gated residual 1,167 -> 1,306.
 //
 // Reference: GpuLinear.enqueue_gemm (gpu/linear.mojo:535-560, c[m, co] =
 // a[m, ci] @ W^T), the MLP's lin0 + gelu_tanh_bias (gpu/linear.mojo:662-684,

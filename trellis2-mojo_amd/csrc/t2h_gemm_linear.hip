@@ -149,7 +149,7 @@ __global__ __launch_bounds__(kThreads, 1) void gemm_kernel(GemmArgs a) {
 // row pieces: half a wave tile's residual is requested before the next tile's
 // operands, the other half while the first is joined. (Reading and writing
 // the f32 residual in the MFMA layout, 32-byte pieces, the out projection of
-// 39,804 tokens took 437 us; so 250.) out may alias res: every element is
+// 39,804 tokens took 409-437 us; so 244-248.) out may alias res: every element is
 // read before it is written, by the same thread.
 template <typename T, typename O, int BT>
 __global__ __launch_bounds__(kThreads, 1) void gemm_res_kernel(GemmArgs a) {
