@@ -129,6 +129,6 @@ def call(name: str, *args) -> None:
     try:
         rc = f(*args)
     except (TypeError, OverflowError):      # ctypes takes more argument forms, and refuses the others its own way
-        rc = getattr(_lib, name)(*args)
+        rc = getattr(load(), name)(*args)
     if rc != T2H_OK:
         check(rc)
