@@ -131,9 +131,10 @@ __device__ __forceinline__ void zip4(const uint32_t (&t)[4], uint32_t* lo, uint3
 // of 16 tokens (E = 8) or of 8 (E = 4), which go to the tile as 16-byte
 // pieces along the tokens: 4 (2) LDS writes and 4 (2) reads per lane and head
 // in place of 32 + 32 (16 + 16) 2-byte ones. With the choice of heads per
-// block below, k alone (12 x 128, f16): 9,000 rows 22.3 -> 19.6 us, 20,000
-// 43.4 -> 31.6, 39,804 59.7 -> 58.0, 150,000 199.7 -> 191.9 (4.8 TB/s); what
-// bounds the large ones is the 128-byte pieces of the strided output planes.
+// block below, k alone (12 x 128, f16): 9,000 rows 22.6 -> 19.8 us, 20,000
+// 44.0 -> 31.7, 39,804 60.0 -> 56.6, 150,000 199.5 -> 192.3 (4.8 TB/s), and
+// 142.7 -> 146.3 at 110,000; what bounds the large ones is the 128-byte pieces
+// of the strided output planes.
 template <int E>
 __device__ __forceinline__ void transpose_to_tile(uint32_t (&w)[kPackIters][E / 2], uint8_t* buf, int wave, int g,
                                                   int m) {
